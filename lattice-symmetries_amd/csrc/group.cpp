@@ -309,9 +309,123 @@ bool group_detect_translations(GroupData &g) {
     g.h_fact_q = q;
     g.h_fact_elem = elem;
     g.h_fact_key = key;
-    return g.d_fact_q.upload(q.data(), q.size()) && g.d_fact_elem.upload(elem.data(), elem.size()) &&
+    g.fact_uniform = g.spin_inversion != -1;
+    for (int e = 0; e < G && g.fact_uniform; ++e)
+      g.fact_uniform = g.h_eig_re[e] == 1.0 && std::memcmp(&g.h_eig_im[e], &g.h_eig_im[0], sizeof(double)) == 0;
+    return group_plan_lines(g, perms) && g.d_fact_q.upload(q.data(), q.size()) && g.d_fact_elem.upload(elem.data(), elem.size()) &&
            g.d_fact_key.upload(key.data(), key.size());
   }
+  return true;
+}
+
+// Point elements of a torus fall into classes {rho o base}: rho runs over the
+// reflections of the torus about row 0 and column 0 (variant bit 0: columns
+// c -> -c, bit 1: rows r -> -r) that the group has.  The rows of rho(base(x))
+// are those of base(x), mirrored and in reversed order, so the two top rows
+// of every translation, reflection and flipped copy of base(x) come from its
+// ly pairs of neighbouring rows.  For a pair P = upper << lx | lower:
+//   line_key[P]   the least value of (top row << lx | next row) among the
+//                 images whose two top rows are this pair: variant, spin flip
+//                 s and rotation a,
+//   line_mask[P]  the images that reach it: bit 8 v + a, v = 4 up + 2 mirror
+//                 + s, where up = 1 takes the pair upside down (rows reversed).
+bool group_plan_lines(GroupData &g, std::vector<Perm> const &perms) {
+  g.line_classes = g.run_points = 0;
+  int const n = g.number_bits, lx = g.fact_lx, ly = g.fact_ly, nq = static_cast<int>(g.h_fact_q.size());
+  if (ly == 1) {
+    if (nq <= kMaxRunPoints) g.run_points = nq;
+    return true;
+  }
+  if (lx < 2 || lx > kMaxLineBits || ly > kMaxLineRows) return true;
+  std::map<Perm, int> point;
+  for (int k = 0; k < nq; ++k) point.emplace(perms[g.h_fact_q[k]], k);
+  auto reflected = [&](Perm const &p, int v) { // rho_v o p: bit i is bit p[rho_v(i)] of x
+    Perm out(n);
+    for (int r = 0; r < ly; ++r)
+      for (int c = 0; c < lx; ++c)
+        out[r * lx + c] = p[((v & 2) ? (ly - r) % ly : r) * lx + ((v & 1) ? (lx - c) % lx : c)];
+    return out;
+  };
+  Perm identity(n);
+  for (int i = 0; i < n; ++i) identity[i] = i;
+  std::vector<int> variants; // a reflection of two rows (columns) is the identity
+  for (int v = 0; v < 4; ++v)
+    if (!((v & 1) && lx == 2) && !((v & 2) && ly == 2) && point.count(reflected(identity, v)) > 0)
+      variants.push_back(v);
+  std::vector<int> order;
+  auto const id = point.find(identity);
+  if (id == point.end()) return true;
+  order.push_back(id->second);
+  for (int k = 0; k < nq; ++k)
+    if (k != id->second) order.push_back(k);
+  std::vector<char> seen(nq, 0);
+  std::vector<int> bases;
+  std::vector<int32_t> line_q;
+  for (int k : order) {
+    if (seen[k]) continue;
+    bases.push_back(k);
+    line_q.resize(line_q.size() + 4, -1);
+    for (int v : variants) {
+      auto const it = point.find(reflected(perms[g.h_fact_q[k]], v));
+      if (it == point.end() || seen[it->second]) return true; // not a union of classes
+      seen[it->second] = 1;
+      line_q[line_q.size() - 4 + v] = it->second;
+    }
+  }
+  int const nc = static_cast<int>(bases.size()), nv = 1 << lx, pairs = 1 << (2 * lx);
+  size_t const base_bytes = static_cast<size_t>(nc - 1) * ly * nv * 8;
+  if (nc * ly > 32 || base_bytes > kMaxLineBaseBytes) return true;
+  // layout: masks, base images, line_q, keys, rotations
+  g.line_off_base = static_cast<size_t>(pairs) * 8;
+  g.line_off_q = g.line_off_base + base_bytes;
+  g.line_off_key = g.line_off_q + static_cast<size_t>(nc) * 16;
+  g.line_off_rot = g.line_off_key + static_cast<size_t>(pairs) * 2;
+  size_t const bytes = g.line_off_rot + static_cast<size_t>(2) * lx * nv;
+  std::vector<uint64_t> buffer((bytes + 7) / 8, 0);
+  auto *const raw = reinterpret_cast<uint8_t *>(buffer.data());
+  auto *const base = reinterpret_cast<uint64_t *>(raw + g.line_off_base);
+  auto *const key = reinterpret_cast<uint16_t *>(raw + g.line_off_key);
+  uint8_t *const rot = raw + g.line_off_rot;
+  std::memcpy(raw + g.line_off_q, line_q.data(), line_q.size() * sizeof(int32_t));
+  uint32_t const rm = static_cast<uint32_t>(nv) - 1;
+  for (int mirror = 0; mirror < 2; ++mirror)
+    for (int v = 0; v < nv; ++v) {
+      uint32_t w = 0;
+      for (int c = 0; c < lx; ++c) w |= ((static_cast<uint32_t>(v) >> (mirror ? (lx - c) % lx : c)) & 1u) << c;
+      for (int a = 0; a < lx; ++a)
+        rot[(mirror * lx + a) * nv + v] = static_cast<uint8_t>(((w >> a) | (w << (lx - a))) & rm);
+    }
+  for (int k = 1; k < nc; ++k) {
+    size_t const e = static_cast<size_t>(g.h_fact_q[bases[k]]) * g.depth;
+    std::vector<uint64_t> const m(g.h_masks.begin() + e, g.h_masks.begin() + e + g.depth);
+    for (int r = 0; r < ly; ++r)
+      for (int v = 0; v < nv; ++v)
+        base[(static_cast<size_t>(k - 1) * ly + r) * nv + v] =
+            apply_network(m, g.h_shifts, static_cast<uint64_t>(v) << (r * lx));
+  }
+  int const flips = g.spin_inversion != 0 ? 2 : 1;
+  for (int p = 0; p < pairs; ++p) {
+    uint32_t const upper = static_cast<uint32_t>(p) >> lx, lower = static_cast<uint32_t>(p) & rm;
+    uint32_t least = ~0u;
+    uint64_t mask = 0;
+    for (int v : variants)
+      for (int s = 0; s < flips; ++s) {
+        uint32_t const x = s ? rm : 0, top = ((v & 2) ? lower : upper) ^ x, next = ((v & 2) ? upper : lower) ^ x;
+        uint8_t const *r = rot + static_cast<size_t>(v & 1) * lx * nv;
+        for (int a = 0; a < lx; ++a) {
+          uint32_t const k = (static_cast<uint32_t>(r[a * nv + top]) << lx) | r[a * nv + next];
+          if (k < least) {
+            least = k;
+            mask = 0;
+          }
+          if (k == least) mask |= uint64_t{1} << (8 * (2 * v + s) + a);
+        }
+      }
+    key[p] = static_cast<uint16_t>(least);
+    buffer[static_cast<size_t>(p)] = mask;
+  }
+  if (!g.d_line.upload(buffer.data(), buffer.size())) return false;
+  g.line_classes = nc;
   return true;
 }
 

@@ -113,6 +113,12 @@ template <typename T> struct DeviceArray {
   }
 };
 
+// What the product has to do with every beta (BatchedOperator.chpl:264-282).
+// The last three are kPermutations through the translation factorisation of
+// the group: state_info_factored, the row-pair search and the run search.
+enum ProjectionKind { kNoProjection = 0, kInversionOnly = 1, kPermutations = 2, kFactored = 3, kLines = 4, kRuns = 5 };
+constexpr bool projects_orbits(int kind) { return kind >= kPermutations; }
+
 // ---------------------------------------------------------------------------
 // Device views
 // ---------------------------------------------------------------------------
@@ -145,6 +151,19 @@ struct GroupView {
   int32_t const *fact_elem;
   int32_t const *fact_key;
   uint64_t fact_m1, fact_m2;
+  // Every character equals that of element 0, flipped copies included (the
+  // symmetric sector), so the element that reaches a minimum does not matter.
+  int fact_uniform;
+  // Row-pair search (line_classes = 0: none; see group_plan_lines).
+  int line_classes;
+  uint16_t const *line_key;   // [2^(2 lx)] least two top rows a pair of rows can give
+  uint64_t const *line_mask;  // [2^(2 lx)] images that give them, bit 8 v + a
+  uint64_t const *line_base;  // [line_classes - 1][ly][2^lx] images of the rows under the class bases
+  uint8_t const *line_rot;    // [2][lx][2^lx] rotations of a row value and of its mirror image
+  int32_t const *line_q;      // [line_classes][4] point element of a class variant
+  // Search over the longest runs of zeros (chains with at most kMaxRunPoints
+  // point elements).
+  int run_points;
 };
 
 // Sorted representatives plus a prefix table over their top bits:
@@ -210,12 +229,25 @@ struct GroupData {
   std::vector<int32_t> h_fact_q, h_fact_elem, h_fact_key;
   DeviceArray<int32_t> d_fact_q, d_fact_elem, d_fact_key;
   uint64_t fact_m1 = 0, fact_m2 = 0;
+  bool fact_uniform = false;
+  // Row-pair search of a torus (group_plan_lines): one buffer with the tables
+  // of GroupView::line_*.
+  int line_classes = 0;
+  DeviceArray<uint64_t> d_line;
+  size_t line_off_base = 0, line_off_q = 0, line_off_key = 0, line_off_rot = 0; // bytes
+  int run_points = 0;
   bool factored() const { return fact_lx > 0 && fermion_species == 0; }
+  bool lines() const { return factored() && line_classes > 0; }
+  bool runs() const { return factored() && run_points > 0; }
   GroupView view() const {
+    auto const *line = reinterpret_cast<uint8_t const *>(d_line.ptr);
     return GroupView{d_masks.ptr, d_eig_re.ptr, d_eig_im.ptr, d_shifts.ptr, size, depth,
                      flip_mask, d_image.ptr, number_bits, norm_eps,
                      fact_lx, fact_ly, static_cast<int>(h_fact_q.size()), d_fact_q.ptr, d_fact_elem.ptr,
-                     d_fact_key.ptr, fact_m1, fact_m2};
+                     d_fact_key.ptr, fact_m1, fact_m2, fact_uniform ? 1 : 0, line_classes,
+                     reinterpret_cast<uint16_t const *>(line + line_off_key), d_line.ptr,
+                     reinterpret_cast<uint64_t const *>(line + line_off_base), line + line_off_rot,
+                     reinterpret_cast<int32_t const *>(line + line_off_q), run_points};
   }
 };
 
@@ -224,6 +256,17 @@ struct GroupData {
 // has real part exactly +-1 (then stabiliser sums are exact in any order).
 // Leaves fact_lx = 0 when the group has no such form.
 bool group_detect_translations(GroupData &g);
+
+// Limits of the row-pair search: a pair of rows indexes the tables, a lane's
+// pairs of all classes fit one 32-bit word, and the class images fit LDS.
+constexpr int kMaxLineBits = 6;
+constexpr int kMaxLineRows = 8;
+constexpr size_t kMaxLineBaseBytes = 16 << 10;
+constexpr int kMaxRunPoints = 2;
+// Tables of the row-pair search for a factorised torus whose point elements
+// fall into classes under row and column reflections, and the run search of a
+// chain (line_classes = run_points = 0 where they do not apply).
+bool group_plan_lines(GroupData &g, std::vector<std::vector<int32_t>> const &perms);
 
 // Marks a group as fermionic (species 1 or 2) and uploads the orbital
 // images; spin inversion must be off.

@@ -227,7 +227,8 @@ template <typename W, int D, int SI, int KIND>
 __device__ __forceinline__ void off_diag_entry(GroupView const &g, OpView const &op,
                                                TermsLds const &l, int k, uint64_t alpha,
                                                double n_alpha, double scale, uint64_t &beta,
-                                               double &c_re, double &c_im, RowTables const *rt) {
+                                               double &c_re, double &c_im,
+                                               OrbitSearch<W, D, SI, KIND> const &search) {
   double const factor = ((__popcll(alpha & l.s[k]) & 1) ? -1.0 : 1.0) * scale;
   double re = l.v[2 * k] * factor, im = l.v[2 * k + 1] * factor;
   beta = alpha ^ l.x[k];
@@ -238,11 +239,11 @@ __device__ __forceinline__ void off_diag_entry(GroupView const &g, OpView const 
       re *= static_cast<double>(SI);
       im *= static_cast<double>(SI);
     }
-  } else if constexpr (KIND == kPermutations || KIND == kFactored) {
+  } else if constexpr (projects_orbits(KIND)) {
     // BatchedOperator.chpl:232-247
-    StateInfo const s =
-        KIND == kFactored ? state_info_factored<W, D, SI>(g, beta, rt) : state_info_one<W, D, SI>(g, beta);
-    double const t_re = (re * s.norm) / n_alpha, t_im = (im * s.norm) / n_alpha;
+    StateInfo const s = search.info(g, beta);
+    double const t_re = (re * s.norm) / n_alpha;
+    double const t_im = im != 0.0 ? (im * s.norm) / n_alpha : im;
     re = s.c_re * t_re - s.c_im * t_im;
     im = s.c_re * t_im + s.c_im * t_re;
     beta = s.rep;
@@ -302,21 +303,21 @@ __global__ __launch_bounds__(256) void otf_push_kernel(GroupView g, OpView op, d
                                                        double *__restrict__ y, int *err, uint64_t *err_state) {
   extern __shared__ uint64_t smem[];
   TermsLds const l = stage_terms(op.off, smem);
-  __shared__ RowTables rt;
-  if constexpr (KIND == kFactored) row_tables_init(g, rt);
+  OrbitSearch<W, D, SI, KIND> search;
+  search.stage(g, smem + 6 * static_cast<size_t>(op.off.count));
   int const T = op.off.count;
   int64_t const i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   bool const valid = i < op.n;
   uint64_t const alpha = valid ? op.idx.reps[i] : 0;
   double const xr = valid ? (CPLX ? x[2 * i] : x[i]) : 0.0;
   double const xi = (CPLX && valid) ? x[2 * i + 1] : 0.0;
-  double const n_alpha = ((KIND == kPermutations || KIND == kFactored) && valid) ? op.norms[i] : 1.0;
+  double const n_alpha = (projects_orbits(KIND) && valid) ? op.norms[i] : 1.0;
   int k = valid ? next_applicable(l, T, alpha, 0) : T;
   while (__any(k < T)) {
     if (k < T) {
       uint64_t beta;
       double c_re, c_im;
-      off_diag_entry<W, D, SI, KIND>(g, op, l, k, alpha, n_alpha, CPLX ? 1.0 : xr, beta, c_re, c_im, &rt);
+      off_diag_entry<W, D, SI, KIND>(g, op, l, k, alpha, n_alpha, CPLX ? 1.0 : xr, beta, c_re, c_im, search);
       bool const nz = CPLX ? (c_re != 0 || c_im != 0) : (c_re != 0);
       if (nz) {
         int64_t const j = op.identity_index ? static_cast<int64_t>(beta) : index_lookup(op.idx, beta);
@@ -337,15 +338,7 @@ __global__ __launch_bounds__(256) void otf_push_kernel(GroupView g, OpView op, d
 // Dispatch over (W, D, SI, KIND): permutation kernels follow the group,
 // the others run on 64-bit words with the spin inversion as SI.
 template <typename F> bool dispatch_op(OperatorCore const &op, F &&f) {
-  if (op.kind == kPermutations) {
-    bool const factored = op.allow_factored && op.group->factored();
-    return dispatch_group(*op.group, [&]<typename W, int D, int SI>() -> bool {
-      if constexpr (SI != kFermionic) {
-        if (factored) return f.template operator()<W, D, SI, kFactored>();
-      }
-      return f.template operator()<W, D, SI, kPermutations>();
-    });
-  }
+  if (op.kind == kPermutations) return dispatch_search(*op.group, op.allow_factored, terms_lds_bytes(op.off.count), f);
   if (op.kind == kInversionOnly) {
     if (op.spin_inversion == 1) return f.template operator()<uint64_t, 0, 1, kInversionOnly>();
     return f.template operator()<uint64_t, 0, -1, kInversionOnly>();
@@ -404,7 +397,6 @@ bool operator_matvec_otf(OperatorCore &op, double const *d_x, double *d_y, bool 
   if (n == 0) return true;
   OpView const v = make_view(op);
   GroupView const g = group_view_or_empty(op);
-  size_t const smem = terms_lds_bytes(op.off.count);
   timer_begin(kTimerOtfF64);
   if (complex_values)
     otf_diag_kernel<true><<<grid_for(n, 256), 256, 0, stream()>>>(v, d_x, d_y, accumulate ? 1 : 0);
@@ -412,6 +404,7 @@ bool operator_matvec_otf(OperatorCore &op, double const *d_x, double *d_y, bool 
     otf_diag_kernel<false><<<grid_for(n, 256), 256, 0, stream()>>>(v, d_x, d_y, accumulate ? 1 : 0);
   LSAMD_HIP(hipGetLastError());
   bool ok = op.off.count == 0 || dispatch_op(op, [&]<typename W, int D, int SI, int KIND>() -> bool {
+    size_t const smem = terms_lds_bytes(op.off.count) + search_lds_bytes<W, D, SI, KIND>(op.group, 256);
     if (complex_values)
       otf_push_kernel<W, D, SI, KIND, true><<<grid_for(n, 256), 256, smem, stream()>>>(
           g, v, d_x, d_y, op.d_err.ptr, op.d_err_state.ptr);
@@ -442,8 +435,8 @@ __global__ __launch_bounds__(256) void csr_fill_kernel(GroupView g, OpView op,
                                                        int *err, uint64_t *err_state) {
   extern __shared__ uint64_t smem[];
   TermsLds const l = stage_terms(op.off, smem);
-  __shared__ RowTables rt;
-  if constexpr (KIND == kFactored) row_tables_init(g, rt);
+  OrbitSearch<W, D, SI, KIND> search;
+  search.stage(g, smem + 6 * static_cast<size_t>(op.off.count));
   int const T = op.off.count;
   int64_t const i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   bool const valid = i < op.n;
@@ -457,7 +450,7 @@ __global__ __launch_bounds__(256) void csr_fill_kernel(GroupView g, OpView op,
     }
     diag[i] = d;
   }
-  double const n_alpha = ((KIND == kPermutations || KIND == kFactored) && valid) ? op.norms[i] : 1.0;
+  double const n_alpha = (projects_orbits(KIND) && valid) ? op.norms[i] : 1.0;
   int64_t o = valid ? row_ptr[i] : 0;
   uint32_t nkept = 0;
   int k = valid ? next_applicable(l, T, alpha, 0) : T;
@@ -465,7 +458,7 @@ __global__ __launch_bounds__(256) void csr_fill_kernel(GroupView g, OpView op,
     if (k < T) {
       uint64_t beta;
       double c_re, c_im;
-      off_diag_entry<W, D, SI, KIND>(g, op, l, k, alpha, n_alpha, 1.0, beta, c_re, c_im, &rt);
+      off_diag_entry<W, D, SI, KIND>(g, op, l, k, alpha, n_alpha, 1.0, beta, c_re, c_im, search);
       uint32_t col = kDropped;
       double val_re = 0.0, val_im = 0.0;
       if (CPLX ? (c_re != 0 || c_im != 0) : (c_re != 0)) {
@@ -918,10 +911,10 @@ bool operator_build_csr(OperatorCore &op, int precision) {
   if (!vals.allocate(static_cast<size_t>(width * (up > 0 ? up : 1)))) return false;
   OpView const v = make_view(op);
   GroupView const g = group_view_or_empty(op);
-  size_t const smem = terms_lds_bytes(op.off.count);
   timer_begin(kTimerCsrBuild);
   if (n > 0) {
     bool ok = dispatch_op(op, [&]<typename W, int D, int SI, int KIND>() -> bool {
+      size_t const smem = terms_lds_bytes(op.off.count) + search_lds_bytes<W, D, SI, KIND>(op.group, 256);
       if (cplx)
         csr_fill_kernel<W, D, SI, KIND, true><<<grid_for(n, 256), 256, smem, stream()>>>(
             g, v, row_ptr.ptr, cols.ptr, vals.ptr, c.diag64.ptr, counts.ptr, op.d_err.ptr,
@@ -1002,272 +995,6 @@ bool operator_build_csr(OperatorCore &op, int precision) {
   if (!op.schedule_set) default_schedule(op);
   LSAMD_HIP(hipStreamSynchronize(stream()));
   return true;
-}
-
-// ---------------------------------------------------------------------------
-// SpMV kernels: LPR lanes share one row
-// ---------------------------------------------------------------------------
-
-template <typename F> bool dispatch_lpr(int lpr, F &&f) {
-  switch (lpr) {
-  case 1: return f.template operator()<1>();
-  case 2: return f.template operator()<2>();
-  case 4: return f.template operator()<4>();
-  case 8: return f.template operator()<8>();
-  case 16: return f.template operator()<16>();
-  case 32: return f.template operator()<32>();
-  case 64: return f.template operator()<64>();
-  default: return fail("lanes per row must be a power of two <= 64");
-  }
-}
-
-// flags: bit 0 non-temporal stream loads, bit 1 die-aware persistent grid
-template <typename F> bool dispatch_flags(int flags, F &&f) {
-  switch (flags & 3) {
-  case 0: return f.template operator()<false, false>();
-  case 1: return f.template operator()<true, false>();
-  case 2: return f.template operator()<false, true>();
-  default: return f.template operator()<true, true>();
-  }
-}
-
-// Grid of a product launch: one workgroup per tile; with the die-aware
-// mapping (flags bit 1) either the persistent grid or, with bit 2, one
-// workgroup per tile rounded up to a multiple of 8, where each workgroup
-// takes one tile of its die's contiguous range.
-int product_grid(OperatorCore const &op, int64_t n, int lpr, int flags) {
-  int const tiles = grid_for(n * lpr, 256);
-  if (flags & 2) return (flags & 4) ? (tiles + 7) / 8 * 8 : op.persistent_blocks;
-  return tiles;
-}
-
-template <typename F> bool dispatch_k(int k, F &&f) {
-  switch (k) {
-  case 1: return f.template operator()<1>();
-  case 2: return f.template operator()<2>();
-  case 4: return f.template operator()<4>();
-  case 8: return f.template operator()<8>();
-  case 16: return f.template operator()<16>();
-  default: return fail("block size must be 1, 2, 4, 8 or 16");
-  }
-}
-
-// The schedule of a block product, by the bytes of x it gathers per stored
-// entry: up to 16 B (FP32 blocks of 1, 2, 4; FP64 blocks of 1, 2) the one
-// tuned on the FP64 vector (8 B), above that the one tuned on the FP32 block
-// of 8 (32 B).  On 6x6 the die-aware full grid that suits the narrow
-// gathers takes the FP32 block of 2 from 6.85 to 6.01 ms, while the block
-// of 8 is fastest on the plain grid.
-struct Schedule {
-  int lanes, flags;
-};
-Schedule block_schedule(OperatorCore const &op, size_t row_bytes) {
-  return row_bytes <= 16 ? Schedule{op.lanes_f64, op.flags_f64} : Schedule{op.lanes_f32, op.flags_f32};
-}
-
-// The FP64 CSR product over `n` rows starting at row_ptr `rp` and output
-// `y` (offsets of the whole arrays; x and the columns stay global).
-bool launch_csr_f64(OperatorCore &op, int64_t const *rp, int64_t n, double const *d_x, double *d_y, int accumulate,
-                    int has_diag) {
-  Csr const &c = op.csr;
-  int const grid = product_grid(op, n, op.lanes_f64, op.flags_f64);
-  return dispatch_lpr(op.lanes_f64, [&]<int LPR>() -> bool {
-    return dispatch_flags(op.flags_f64, [&]<bool NT, bool DIE>() -> bool {
-      if (c.wide)
-        csr_f64_wide_kernel<LPR, NT, DIE><<<grid, 256, sizeof(double) * c.table_size, stream()>>>(
-            n, rp, c.cols.ptr, c.vidx.ptr, c.table64.ptr, c.table_size, c.diag64.ptr, d_x, d_y, accumulate, has_diag);
-      else if (c.packed)
-        csr_f64_kernel<LPR, NT, DIE, true><<<grid, 256, 0, stream()>>>(
-            n, rp, c.cols.ptr, nullptr, c.table64.ptr, c.table_size, c.diag64.ptr, d_x, d_y, accumulate, has_diag);
-      else
-        csr_f64_kernel<LPR, NT, DIE, false><<<grid, 256, 0, stream()>>>(
-            n, rp, c.cols.ptr, c.vals64.ptr, nullptr, 0, c.diag64.ptr, d_x, d_y, accumulate, has_diag);
-      LSAMD_HIP(hipGetLastError());
-      return true;
-    });
-  });
-}
-
-bool operator_csr_f64(OperatorCore &op, double const *d_x, double *d_y, bool accumulate) {
-  Csr const &c = op.csr;
-  if (c.is_complex) return fail("the CSR holds complex values: use a sector batch for its products");
-  if (!c.has64) return fail("FP64 CSR has not been built");
-  int64_t const n = c.rows;
-  if (n == 0) return true;
-  timer_begin(kTimerCsrF64);
-  bool const ok = launch_csr_f64(op, c.row_ptr.ptr, n, d_x, d_y, accumulate ? 1 : 0, op.diag.count > 0 ? 1 : 0);
-  timer_end(kTimerCsrF64);
-  return ok;
-}
-
-__global__ __launch_bounds__(256) void diag_times_kernel(int64_t n, double const *__restrict__ diag,
-                                                         double const *__restrict__ x, double *__restrict__ y) {
-  int64_t const i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (i < n) y[i] = diag[i] * x[i];
-}
-
-bool operator_csr_f64_diag(OperatorCore &op, double const *d_x, double *d_y) {
-  Csr const &c = op.csr;
-  if (c.is_complex || !c.has64) return fail("FP64 CSR has not been built");
-  if (c.rows == 0) return true;
-  diag_times_kernel<<<grid_for(c.rows, 256), 256, 0, stream()>>>(c.rows, c.diag64.ptr, d_x, d_y);
-  LSAMD_HIP(hipGetLastError());
-  return true;
-}
-
-bool operator_csr_f64_rows(OperatorCore &op, double const *d_x, double *d_y, int64_t r0, int64_t r1) {
-  Csr const &c = op.csr;
-  if (c.is_complex || !c.has64) return fail("FP64 CSR has not been built");
-  if (r0 < 0 || r1 > c.rows || r0 > r1) return fail("row range outside the CSR");
-  if (r1 == r0) return true;
-  return launch_csr_f64(op, c.row_ptr.ptr + r0, r1 - r0, d_x, d_y + r0, 1, 0);
-}
-
-bool operator_csr_f32_block(OperatorCore &op, int k, float const *d_x, float *d_y) {
-  Csr const &c = op.csr;
-  if (c.is_complex) return fail("the CSR holds complex values: use a sector batch for its products");
-  if (!c.has32) return fail("FP32 CSR has not been built");
-  int64_t const n = c.rows;
-  if (n == 0) return true;
-  Schedule const s = block_schedule(op, sizeof(float) * static_cast<size_t>(k));
-  timer_begin(kTimerCsrF32);
-  bool ok = dispatch_k(k, [&]<int K>() -> bool {
-    return dispatch_lpr(s.lanes, [&]<int LPR>() -> bool {
-      int const grid = product_grid(op, n, LPR, s.flags);
-      return dispatch_flags(s.flags, [&]<bool NT, bool DIE>() -> bool {
-        if (c.wide)
-          csr_block_wide_kernel<K, LPR, float, float, NT, DIE><<<grid, 256, sizeof(float) * c.table_size, stream()>>>(
-              n, c.row_ptr.ptr, c.cols.ptr, c.vidx.ptr, c.table32.ptr, c.table_size, c.diag32.ptr, d_x, d_y);
-        else if (c.packed)
-          csr_block_kernel<K, LPR, float, float, NT, DIE, true><<<grid, 256, 0, stream()>>>(
-              n, c.row_ptr.ptr, c.cols.ptr, nullptr, c.table32.ptr, c.table_size, c.diag32.ptr, d_x, d_y);
-        else
-          csr_block_kernel<K, LPR, float, float, NT, DIE, false><<<grid, 256, 0, stream()>>>(
-              n, c.row_ptr.ptr, c.cols.ptr, c.vals32.ptr, nullptr, 0, c.diag32.ptr, d_x, d_y);
-        LSAMD_HIP(hipGetLastError());
-        return true;
-      });
-    });
-  });
-  timer_end(kTimerCsrF32);
-  return ok;
-}
-
-bool operator_csr_f64_block(OperatorCore &op, int k, double const *d_x, double *d_y) {
-  Csr const &c = op.csr;
-  if (c.is_complex) return fail("the CSR holds complex values: use a sector batch for its products");
-  if (!c.has64) return fail("FP64 CSR has not been built");
-  int64_t const n = c.rows;
-  if (n == 0) return true;
-  Schedule const s = block_schedule(op, sizeof(double) * static_cast<size_t>(k));
-  timer_begin(kTimerCsrF64Block);
-  bool ok = dispatch_k(k, [&]<int K>() -> bool {
-    return dispatch_lpr(s.lanes, [&]<int LPR>() -> bool {
-      int const grid = product_grid(op, n, LPR, s.flags);
-      return dispatch_flags(s.flags, [&]<bool NT, bool DIE>() -> bool {
-        if (c.wide)
-          csr_block_wide_kernel<K, LPR, double, double, NT, DIE><<<grid, 256, sizeof(double) * c.table_size,
-                                                                   stream()>>>(
-              n, c.row_ptr.ptr, c.cols.ptr, c.vidx.ptr, c.table64.ptr, c.table_size, c.diag64.ptr, d_x, d_y);
-        else if (c.packed)
-          csr_block_kernel<K, LPR, double, double, NT, DIE, true><<<grid, 256, 0, stream()>>>(
-              n, c.row_ptr.ptr, c.cols.ptr, nullptr, c.table64.ptr, c.table_size, c.diag64.ptr, d_x, d_y);
-        else
-          csr_block_kernel<K, LPR, double, double, NT, DIE, false><<<grid, 256, 0, stream()>>>(
-              n, c.row_ptr.ptr, c.cols.ptr, c.vals64.ptr, nullptr, 0, c.diag64.ptr, d_x, d_y);
-        LSAMD_HIP(hipGetLastError());
-        return true;
-      });
-    });
-  });
-  timer_end(kTimerCsrF64Block);
-  return ok;
-}
-
-// Times every product schedule (lanes per row x stream-load kind x grid
-// mapping) on the cached matrix and keeps the fastest, separately for the
-// FP64 kernel and the FP32 block-of-8 kernel: the schedules of the narrow
-// and the wide gathers (block_schedule).
-// plain, non-temporal, die-aware persistent (with / without non-temporal),
-// die-aware over the full grid (with / without non-temporal)
-constexpr int kScheduleFlags[] = {0, 1, 2, 3, 6, 7};
-
-int operator_autotune(OperatorCore &op) {
-  Csr const &c = op.csr;
-  int64_t const n = c.rows;
-  if (n == 0 || c.is_complex) return op.lanes_f64;
-  op.schedule_set = true;
-  hipDeviceProp_t prop;
-  int dev = 0;
-  if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess) {
-    // four workgroups per CU; with the wide table as many as fit beside their
-    // LDS copies of it (up to eight), so each CU stages the table a few times
-    int per_cu = 4;
-    if (c.wide)
-      per_cu = static_cast<int>(std::min<size_t>(
-          8, std::max<size_t>(1, (160u << 10) / (sizeof(double) * static_cast<size_t>(c.table_size)))));
-    op.persistent_blocks = std::max(8, (prop.multiProcessorCount * per_cu / 8) * 8);
-  }
-  int const cand[] = {2, 4, 8, 16, 32, 64};
-  hipEvent_t e0, e1;
-  (void)hipEventCreate(&e0);
-  (void)hipEventCreate(&e1);
-  auto time_it = [&](auto &&launch) -> float {
-    launch();
-    (void)hipEventRecord(e0, stream());
-    for (int r = 0; r < 3; ++r) launch();
-    (void)hipEventRecord(e1, stream());
-    (void)hipEventSynchronize(e1);
-    float ms = 0;
-    (void)hipEventElapsedTime(&ms, e0, e1);
-    return ms;
-  };
-  if (c.has64) {
-    DeviceArray<double> x, y;
-    if (x.allocate(n) && y.allocate(n)) {
-      (void)hipMemsetAsync(x.ptr, 0, sizeof(double) * n, stream());
-      float best = 1e30f;
-      int best_l = op.lanes_f64, best_f = op.flags_f64;
-      for (int f : kScheduleFlags)
-        for (int l : cand) {
-          op.lanes_f64 = l;
-          op.flags_f64 = f;
-          float const ms = time_it([&] { (void)operator_csr_f64(op, x.ptr, y.ptr, false); });
-          if (ms < best) {
-            best = ms;
-            best_l = l;
-            best_f = f;
-          }
-        }
-      op.lanes_f64 = best_l;
-      op.flags_f64 = best_f;
-    }
-  }
-  if (c.has32) {
-    DeviceArray<float> x, y;
-    if (x.allocate(static_cast<size_t>(n) * 8) && y.allocate(static_cast<size_t>(n) * 8)) {
-      (void)hipMemsetAsync(x.ptr, 0, sizeof(float) * n * 8, stream());
-      float best = 1e30f;
-      int best_l = op.lanes_f32, best_f = op.flags_f32;
-      for (int f : kScheduleFlags)
-        for (int l : cand) {
-          op.lanes_f32 = l;
-          op.flags_f32 = f;
-          float const ms = time_it([&] { (void)operator_csr_f32_block(op, 8, x.ptr, y.ptr); });
-          if (ms < best) {
-            best = ms;
-            best_l = l;
-            best_f = f;
-          }
-        }
-      op.lanes_f32 = best_l;
-      op.flags_f32 = best_f;
-    }
-  }
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
-  (void)hipStreamSynchronize(stream());
-  return op.lanes_f64;
 }
 
 } // namespace lsamd

@@ -23,11 +23,6 @@ struct Terms {
   uint64_t fingerprint() const;
 };
 
-// What the product has to do with every beta (BatchedOperator.chpl:264-282).
-// kFactored: kPermutations through the translation factorisation of the
-// group (state_info_factored).
-enum ProjectionKind { kNoProjection = 0, kInversionOnly = 1, kPermutations = 2, kFactored = 3 };
-
 struct Csr {
   int64_t rows = 0;
   int64_t nnz = 0;

@@ -12,9 +12,8 @@
 
 namespace lsamd {
 
-// FACT: through the translation factorisation of the group (state_info_factored,
-// bit for bit the same results) instead of element by element.
-template <typename W, int D, int SI, bool FACT>
+// KIND: the orbit search (dispatch_search); every kind gives the same bits.
+template <typename W, int D, int SI, int KIND>
 __global__ __launch_bounds__(256) void state_info_kernel(GroupView g, int64_t count,
                                                          uint64_t const *__restrict__ xs,
                                                          int64_t x_stride,
@@ -22,15 +21,12 @@ __global__ __launch_bounds__(256) void state_info_kernel(GroupView g, int64_t co
                                                          int64_t rep_stride,
                                                          double *__restrict__ chars,
                                                          double *__restrict__ norms) {
-  __shared__ RowTables rt;
-  if constexpr (FACT) row_tables_init(g, rt);
+  extern __shared__ uint64_t search_lds[];
+  OrbitSearch<W, D, SI, KIND> search;
+  search.stage(g, search_lds);
   int64_t const i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= count) return;
-  StateInfo s;
-  if constexpr (FACT)
-    s = state_info_factored<W, D, SI>(g, xs[i * x_stride], &rt);
-  else
-    s = state_info_one<W, D, SI>(g, xs[i * x_stride]);
+  StateInfo const s = search.info(g, xs[i * x_stride]);
   reps[i * rep_stride] = s.rep;
   chars[2 * i] = s.c_re;
   chars[2 * i + 1] = s.c_im;
@@ -56,16 +52,9 @@ bool launch_state_info(GroupData const &g, int64_t count, uint64_t const *d_x, i
                        uint64_t *d_reps, int64_t rep_stride, double *d_chars, double *d_norms) {
   if (count <= 0) return true;
   GroupView const v = g.view();
-  return dispatch_group(g, [&]<typename W, int D, int SI>() -> bool {
-    if constexpr (SI != kFermionic) {
-      if (g.factored()) {
-        state_info_kernel<W, D, SI, true><<<grid_for(count, 256), 256, 0, stream()>>>(
-            v, count, d_x, x_stride, d_reps, rep_stride, d_chars, d_norms);
-        LSAMD_HIP(hipGetLastError());
-        return true;
-      }
-    }
-    state_info_kernel<W, D, SI, false><<<grid_for(count, 256), 256, 0, stream()>>>(
+  return dispatch_search(g, true, 0, [&]<typename W, int D, int SI, int KIND>() -> bool {
+    size_t const smem = search_lds_bytes<W, D, SI, KIND>(&g, 256);
+    state_info_kernel<W, D, SI, KIND><<<grid_for(count, 256), 256, smem, stream()>>>(
         v, count, d_x, x_stride, d_reps, rep_stride, d_chars, d_norms);
     LSAMD_HIP(hipGetLastError());
     return true;
