@@ -250,6 +250,7 @@ std::shared_ptr<CachedOperator> cached_operator(ls_hs_operator const *op) {
   char const *mode = std::getenv("LSAMD_MATVEC");
   size_t free_b = 0, total_b = 0;
   (void)hipMemGetInfo(&free_b, &total_b);
+  free_b += pool_cached_bytes();
   double const estimate = static_cast<double>(c->core.number_states) *
                           std::max(1, c->core.off.count) * 12.0;
   c->use_csr = mode != nullptr ? std::strcmp(mode, "csr") == 0 : estimate < 0.4 * static_cast<double>(free_b);
@@ -651,6 +652,7 @@ extern "C" void ls_chpl_finalize(void) {
     g_op_cache.clear();
   }
   release_enumeration_scratch();
+  pool_trim();
 }
 
 extern "C" void ls_amd_forget_operator(ls_hs_operator const *op) {

@@ -1,8 +1,11 @@
 // device.cpp -- device set-up, stream, timers, errors and the device-memory
 // helpers of the additive ABI.
+#include <algorithm>
 #include <atomic>
 #include <cstdlib>
 #include <cstring>
+#include <map>
+#include <unordered_map>
 
 #include "lsamd_internal.hpp"
 
@@ -76,6 +79,113 @@ void timer_end(int family) {
   if (family < 0 || family >= kTimerCount || !g_device_ready) return;
   (void)hipEventRecord(g_ev_end[family], g_stream);
   g_ev_used[family] = true;
+}
+
+// ---------------------------------------------------------------------------
+// Block pool.  The driver clears the pages of freed device memory before it
+// hands them out again, at about 35 GB/s: a program that builds one operator
+// after another (38 GB of temporaries and results on the 6x6 lattice) waited
+// 0.8 s per build for that, and a call on a small host batch spent most of
+// its time in hipMalloc / hipFree.  A block is released only after the whole
+// device has finished (as hipFree does), so whatever stream still used it is
+// done when it is handed out again.
+// ---------------------------------------------------------------------------
+namespace {
+
+struct BlockPool {
+  std::mutex mutex;
+  std::unordered_map<void *, size_t> live;
+  struct Free {
+    void *ptr;
+    uint64_t stamp;
+  };
+  std::multimap<size_t, Free> free; // by size
+  size_t cached = 0, capacity = 0;
+  uint64_t clock = 0;
+
+  // Called with the mutex held: down to `limit` cached bytes.
+  void shrink(size_t limit) {
+    while (cached > limit && !free.empty()) {
+      auto oldest = free.begin();
+      for (auto it = free.begin(); it != free.end(); ++it)
+        if (it->second.stamp < oldest->second.stamp) oldest = it;
+      (void)hipFree(oldest->second.ptr);
+      cached -= oldest->first;
+      free.erase(oldest);
+    }
+  }
+};
+
+// Never destroyed: arrays of static duration are released at process exit.
+BlockPool &pool() {
+  static BlockPool *const p = new BlockPool;
+  return *p;
+}
+
+size_t block_size(size_t bytes) {
+  size_t const unit = bytes < (size_t{1} << 20) ? 256 : (bytes < (size_t{64} << 20) ? size_t{64} << 10 : size_t{2} << 20);
+  return (bytes + unit - 1) / unit * unit;
+}
+
+// LSAMD_POOL_BYTES, or a twelfth of the device's memory.
+size_t pool_capacity() {
+  if (char const *e = std::getenv("LSAMD_POOL_BYTES")) return static_cast<size_t>(std::strtoull(e, nullptr, 10));
+  size_t free_b = 0, total_b = 0;
+  (void)hipMemGetInfo(&free_b, &total_b);
+  return total_b / 12;
+}
+
+} // namespace
+
+void *pool_allocate(size_t bytes) {
+  size_t const want = block_size(bytes);
+  BlockPool &p = pool();
+  std::lock_guard<std::mutex> lock(p.mutex);
+  void *ptr = nullptr;
+  auto const it = p.free.lower_bound(want);
+  size_t size = want;
+  if (it != p.free.end() && it->first - want <= want / 8) {
+    ptr = it->second.ptr;
+    size = it->first;
+    p.cached -= size;
+    p.free.erase(it);
+  } else if (hipMalloc(&ptr, want) != hipSuccess) {
+    (void)hipGetLastError();
+    p.shrink(0);
+    if (hipMalloc(&ptr, want) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+  }
+  p.live[ptr] = size;
+  return ptr;
+}
+
+void pool_release(void *ptr) {
+  bool const idle = hipDeviceSynchronize() == hipSuccess;
+  BlockPool &p = pool();
+  std::lock_guard<std::mutex> lock(p.mutex);
+  auto const it = p.live.find(ptr);
+  size_t const size = it->second;
+  p.live.erase(it);
+  if (p.capacity == 0) p.capacity = std::max<size_t>(1, pool_capacity());
+  if (!idle || size > p.capacity) {
+    (void)hipFree(ptr);
+    return;
+  }
+  p.free.emplace(size, BlockPool::Free{ptr, ++p.clock});
+  p.cached += size;
+  p.shrink(p.capacity);
+}
+
+void pool_trim() {
+  std::lock_guard<std::mutex> lock(pool().mutex);
+  pool().shrink(0);
+}
+
+size_t pool_cached_bytes() {
+  std::lock_guard<std::mutex> lock(pool().mutex);
+  return pool().cached;
 }
 
 } // namespace lsamd

@@ -70,6 +70,15 @@ enum TimerFamily {
 void timer_begin(int family);
 void timer_end(int family);
 
+// Device memory for DeviceArray.  Freed blocks are kept for later allocations
+// of nearly their size (device.cpp), up to pool_capacity() bytes together;
+// the least recently freed go back to the driver first, and all of them when
+// an allocation fails and on ls_chpl_finalize.
+void *pool_allocate(size_t bytes); // null when the device is out of memory
+void pool_release(void *ptr);
+void pool_trim();
+size_t pool_cached_bytes();
+
 // RAII device buffer.
 template <typename T> struct DeviceArray {
   T *ptr = nullptr;
@@ -95,8 +104,8 @@ template <typename T> struct DeviceArray {
   bool allocate(size_t n) {
     reset();
     if (n == 0) return true;
-    if (hipMalloc(reinterpret_cast<void **>(&ptr), n * sizeof(T)) != hipSuccess) {
-      ptr = nullptr;
+    ptr = static_cast<T *>(pool_allocate(n * sizeof(T)));
+    if (ptr == nullptr) {
       return fail("hipMalloc of " + std::to_string(n * sizeof(T)) + " bytes failed");
     }
     count = n;
@@ -107,7 +116,7 @@ template <typename T> struct DeviceArray {
     return copy_to_device(ptr, host, n * sizeof(T));
   }
   void reset() {
-    if (ptr != nullptr) (void)hipFree(ptr);
+    if (ptr != nullptr) pool_release(ptr);
     ptr = nullptr;
     count = 0;
   }
