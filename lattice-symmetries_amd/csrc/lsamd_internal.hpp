@@ -192,6 +192,7 @@ struct TermsView {
   uint64_t const *r;
   uint64_t const *x;
   uint64_t const *s;
+  uint64_t const *actions; // [count][4]: x, s, v (re, im)
   int count;
 };
 

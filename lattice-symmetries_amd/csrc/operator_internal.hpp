@@ -16,9 +16,10 @@ struct Terms {
   std::vector<uint64_t> h_m, h_r, h_x, h_s;
   DeviceArray<double> d_v;
   DeviceArray<uint64_t> d_m, d_r, d_x, d_s;
+  DeviceArray<uint64_t> d_actions; // per term: x, s, v (re, im), in one 32-byte record
   bool load(ls_hs_nonbranching_terms const *t);
   TermsView view() const {
-    return TermsView{d_v.ptr, d_m.ptr, d_r.ptr, d_x.ptr, d_s.ptr, count};
+    return TermsView{d_v.ptr, d_m.ptr, d_r.ptr, d_x.ptr, d_s.ptr, d_actions.ptr, count};
   }
   uint64_t fingerprint() const;
 };

@@ -510,6 +510,7 @@ template <typename W, int SI> struct LineSearch {
   __device__ __forceinline__ OrbitMinimum<W, SI> minimum(GroupView const &g, W x) const {
     int const lx = g.fact_lx, ly = g.fact_ly, top = (ly - 1) * lx;
     uint32_t const rm = (1u << lx) - 1, pm = (1u << (2 * lx)) - 1;
+    W const all = static_cast<W>(g.flip);
     uint32_t least = ~0u, hits = 0; // bit c * ly + j: pair j of class c reaches it
     for (int c = 0; c < g.line_classes; ++c) {
       W y = x;
@@ -546,15 +547,19 @@ template <typename W, int SI> struct LineSearch {
       int const bit = __ffsll(static_cast<unsigned long long>(mask)) - 1;
       mask &= mask - 1;
       int const a = bit & 7, s = (bit >> 3) & 1, v = bit >> 4; // v: mirrored + 2 * upside down
-      int row = (v & 2) ? j : (j + 1 == ly ? 0 : j + 1);
-      int const at = (v & 2) && row != 0 ? ly - row : row; // the top row's place in the point element's image
+      bool const up = (v & 2) != 0;
+      int const row = up ? j : (j + 1 == ly ? 0 : j + 1); // of y, the image's top row
+      int const at = up && row != 0 ? ly - row : row;     // its place in the point element's image
       uint8_t const *rt = rot + (((v & 1) * lx + a) << lx);
-      uint32_t const flip = s ? rm : 0u;
+      // y flipped and turned so that its rows run from the image's top row
+      // down (or up, upside down): the rows below it first
+      W z = s ? static_cast<W>(y ^ all) : y;
+      int const turn = (up ? row : (row + 1 == ly ? 0 : row + 1)) * lx;
+      z = turn == 0 ? z : static_cast<W>(((z & all) >> turn) | ((z << (g.nbits - turn)) & all));
       W w = 0;
-      for (int i = 0; i < ly; ++i) {
-        w = static_cast<W>(w << lx) | rt[(static_cast<uint32_t>(y >> (row * lx)) & rm) ^ flip];
-        row = (v & 2) ? (row + 1 == ly ? 0 : row + 1) : (row == 0 ? ly - 1 : row - 1);
-      }
+#pragma unroll
+      for (int i = 0; i < kMaxLineRows; ++i)
+        if (i < ly) w = static_cast<W>(w << lx) | rt[static_cast<uint32_t>(z >> (up ? i * lx : top - i * lx)) & rm];
       int const k = g.fact_uniform ? 0 : (g.line_q[4 * c + v] * ly + (at + 1 == ly ? 0 : at + 1)) * lx + a;
       out.visit(g, w, k, s);
     }

@@ -1,0 +1,81 @@
+"""The value-table CSR build (targets counted and placed by the fill pass)
+against the general build: the same rows, columns, values and products, at
+the edges of its formats -- 256 and 257 distinct values, rows of one entry to
+more than the register sort takes, a target row too long for its place bits,
+and rows of a wave that end inside it."""
+import numpy as np
+import pytest
+
+import lsamd
+from lsamd import models
+from lsamd.expr import Expr, Term, sigma_minus, sigma_plus, sum_exprs
+
+pytestmark = pytest.mark.gpu
+
+
+def basis(n, weight=None, group=False, inversion=None):
+    S = None
+    if group:
+        S = lsamd.Symmetries([lsamd.Symmetry(models.chain_translation(n), 0), lsamd.Symmetry(models.chain_parity(n), 0)])
+    b = lsamd.DeviceBasis(n, weight, inversion, S)
+    b.build()
+    return b
+
+
+def fields(n, couplings):
+    return sum_exprs((sigma_plus(i) + sigma_minus(i)) * c for i, c in zip(range(n), couplings))
+
+
+def collective(n):
+    """Every state of one flipped spin goes to |0...01>: row 0 gets them all."""
+    return sum_exprs(sigma_minus(i) * sigma_plus(0) * (1.0 + (i % 3)) for i in range(1, n))
+
+
+CASES = {
+    "chain16": lambda: (basis(16, 8, True, 1), models.j1j2_chain(16)),
+    "chain13": lambda: (basis(13, 5, True), models.j1j2_chain(13)),
+    "chain9-all": lambda: (basis(9), models.heisenberg_chain(9)),
+    "field12": lambda: (basis(12), fields(12, [0.5 + i for i in range(12)])),
+    "two-states": lambda: (basis(2, 1), models.heisenberg_chain(2)),
+    "values256": lambda: (basis(24, 2), pair_hops(24, 128)),
+    "values257": lambda: (basis(24, 2), pair_hops(24, 129)),
+    "collective60": lambda: (basis(60, 1), collective(60)),
+    "flips300": lambda: (basis(10), all_flips(10, 300)),
+    "flips1023": lambda: (basis(10), all_flips(10, 1023)),
+    "flips4500": lambda: (basis(13), all_flips(13, 4500)),
+}
+
+
+def pair_hops(n, count):
+    """`count` hops with couplings of their own, both directions: 2 x count values at most."""
+    pairs = [(i, j) for i in range(n) for j in range(i + 1, n)][:count]
+    return sum_exprs(sigma_plus(i) * sigma_minus(j) * (1.0 + 0.25 * k) + sigma_plus(j) * sigma_minus(i) * (-1.0 - 0.25 * k)
+                     for k, (i, j) in enumerate(pairs))
+
+
+def all_flips(n, count):
+    """Flips of `count` subsets of the sites: rows of `count` entries."""
+    out = {}
+    for mask in range(1, count + 1):
+        t = Term(0.5 + mask % 7, 0, 0, 0, mask, 0)
+        out[(t.m, t.l, t.r, t.x, t.s)] = t.v
+    return Expr(out)
+
+
+@pytest.mark.parametrize("name", CASES)
+def test_table_build_equals_the_general_build(engine, name):
+    b, expr = CASES[name]()
+    print(name, b.number_states, flush=True)
+    table, plain = lsamd.DeviceOperator(b, expr), lsamd.DeviceOperator(b, expr)
+    plain.set_csr_packing(False)
+    assert table.build_csr(96) == plain.build_csr(96)
+    for got, want in zip(table.csr_arrays(), plain.csr_arrays()):
+        assert np.array_equal(got, want)
+    x = np.random.default_rng(1).standard_normal(b.number_states)
+    assert np.array_equal(table.matvec(x, "csr"), plain.matvec(x, "csr"))
+    # the fused product adds a row's L entries in another order: each of the L
+    # sums rounds by at most eps times the sum of L products
+    longest = 1 + np.diff(plain.csr_arrays()[0]).max(initial=0)
+    scale = max(np.abs(a).max(initial=0) for a in plain.csr_arrays()[2:]) * np.abs(x).max()
+    bound = np.finfo(float).eps * longest ** 2 * scale
+    assert np.abs(table.matvec(x, "otf") - plain.matvec(x, "csr")).max() <= bound
