@@ -92,21 +92,36 @@ bool launch_state_index(IndexView const &idx, int64_t count, uint64_t const *d_x
   return true;
 }
 
-// offsets[b] = first position whose state has prefix >= b (b = 0 .. 2^P).
+// offsets[b] = first position whose state has prefix >= b (b = 0 .. 2^P).  A
+// workgroup owns kPrefixBlock entries: one thread each searches the whole list
+// for its first and its end, and the entries between search only what lies
+// between those two (nothing, for the many prefixes no representative has).
+// 6x6 (2^26 entries): 0.75 ms with every entry searching the list.
+constexpr int kPrefixBlock = 1024;
+
+__device__ __forceinline__ int64_t first_with_prefix(uint64_t const *__restrict__ reps, int64_t lo, int64_t n, int shift,
+                                                     uint64_t b) {
+  while (n > 0) {
+    int64_t const half = n >> 1;
+    bool const less = (reps[lo + half] >> shift) < b;
+    lo = less ? lo + half + 1 : lo;
+    n = less ? n - half - 1 : half;
+  }
+  return lo;
+}
+
 __global__ __launch_bounds__(256) void prefix_table_kernel(uint64_t const *__restrict__ reps,
                                                            int64_t count, int shift,
                                                            int64_t table_size,
                                                            uint32_t *__restrict__ offsets) {
-  int64_t const b = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (b > table_size) return;
-  int64_t lo = 0, n = count;
-  while (n > 0) {
-    int64_t const half = n >> 1;
-    bool const less = (reps[lo + half] >> shift) < static_cast<uint64_t>(b);
-    lo = less ? lo + half + 1 : lo;
-    n = less ? n - half - 1 : half;
-  }
-  offsets[b] = static_cast<uint32_t>(lo);
+  __shared__ int64_t ends[2];
+  int64_t const b0 = static_cast<int64_t>(blockIdx.x) * kPrefixBlock;
+  if ((threadIdx.x & 63) == 0 && threadIdx.x < 128)
+    ends[threadIdx.x >> 6] =
+        first_with_prefix(reps, 0, count, shift, static_cast<uint64_t>(b0 + (threadIdx.x >> 6) * kPrefixBlock));
+  __syncthreads();
+  for (int64_t b = b0 + threadIdx.x; b < b0 + kPrefixBlock && b <= table_size; b += 256)
+    offsets[b] = static_cast<uint32_t>(first_with_prefix(reps, ends[0], ends[1] - ends[0], shift, static_cast<uint64_t>(b)));
 }
 
 int default_prefix_bits(int number_bits, int64_t count) {
@@ -134,7 +149,7 @@ bool index_build(IndexData &idx, uint64_t const *d_reps, int64_t count, int numb
   idx.d_reps = d_reps;
   int64_t const table_size = int64_t{1} << prefix_bits;
   if (!idx.d_offsets.allocate(static_cast<size_t>(table_size + 1))) return false;
-  prefix_table_kernel<<<grid_for(table_size + 1, 256), 256, 0, stream()>>>(
+  prefix_table_kernel<<<grid_for(table_size + 1, kPrefixBlock), 256, 0, stream()>>>(
       d_reps, count, idx.shift, table_size, idx.d_offsets.ptr);
   LSAMD_HIP(hipGetLastError());
   LSAMD_HIP(hipStreamSynchronize(stream()));
