@@ -656,6 +656,263 @@ bool exclusive_scan(uint32_t const *d_counts, int64_t n, uint64_t *d_offsets, ui
 }
 
 // ---------------------------------------------------------------------------
+// Split enumeration for tori with the row-pair search (GroupView::line_*) and
+// a fixed Hamming weight.
+//
+// A representative's top row is the least row that any image can have, so
+// every row of it has least image row >= its top row.  A state is split into
+// its upper rows `high` and its lower rows `low`: an admissible high is its
+// own least top row, with rows and row pairs of its own that do not fall below
+// its top ones, and the lows that go with it are those of the remaining weight
+// whose rows pass against the top row, listed once per top row and weight.
+// On 6x6 this leaves about one candidate in twenty of the fixed-weight states
+// (before: 4.5 G states, each stepped to by Gosper's rule and tested against
+// its translations), and a candidate costs a list read and one table lookup
+// per row pair.  Its survivors (the two top rows are the least pair of the
+// first class) queue up for the full search.  Candidates run in ascending
+// order, so acceptance bits, a scan over tiles and a second pass that writes
+// keep the list ascending.
+// 6x6 basis: 26.7 -> 3.2 ms; the count pass takes 1.9 ms, bound by VALU work and
+// the search's LDS lookups.
+// ---------------------------------------------------------------------------
+
+constexpr int kSplitTile = 2048; // candidates of a workgroup
+constexpr int kMaxSplitLow = 18; // bits of the lower rows
+constexpr int kMaxSplitHigh = 24;
+
+struct SplitView {
+  uint32_t const *lists;  // lows
+  uint32_t const *starts; // [2^lx][kMaxSplitLow + 2] first entry by top row and weight
+  uint32_t const *highs;  // admissible highs with a non-empty list, ascending
+  uint64_t const *first;  // [count + 1] first candidate of a high
+  int64_t count, total;   // highs, candidates
+  uint64_t lower, upper;  // states outside are left out
+  int low_rows, hamming;
+};
+
+__device__ __forceinline__ uint32_t least_row(GroupView const &g, uint32_t v) {
+  return g.line_key[v << g.fact_lx | v] >> g.fact_lx;
+}
+
+// Lists the lows of top row tops[blockIdx.x] and weight blockIdx.y, ascending.
+__global__ __launch_bounds__(1024) void split_lists_kernel(GroupView g, int low_rows, uint32_t const *__restrict__ tops,
+                                                           uint32_t const *__restrict__ starts,
+                                                           uint32_t *__restrict__ lists) {
+  __shared__ uint32_t s_wave[16];
+  uint32_t const top = tops[blockIdx.x];
+  int const w = static_cast<int>(blockIdx.y), lane = static_cast<int>(threadIdx.x) & 63, wave = static_cast<int>(threadIdx.x) >> 6;
+  uint32_t const *st = starts + top * (kMaxSplitLow + 2);
+  if (st[w] == st[w + 1]) return;
+  uint32_t const rm = (1u << g.fact_lx) - 1, all = 1u << (low_rows * g.fact_lx);
+  uint32_t at = st[w];
+  for (uint32_t v0 = 0; v0 < all; v0 += 4 * 1024) {
+    uint32_t ok = 0; // four neighbouring values to a thread
+    for (uint32_t q = 0; q < 4; ++q) {
+      uint32_t const v = v0 + 4 * threadIdx.x + q;
+      bool on = v < all && __popc(v) == w;
+      for (int r = 0; r < low_rows && on; ++r) on = least_row(g, v >> (r * g.fact_lx) & rm) >= top;
+      ok |= (on ? 1u : 0u) << q;
+    }
+    uint32_t sum = static_cast<uint32_t>(__popc(ok));
+    for (int off = 1; off < 64; off <<= 1) {
+      uint32_t const up = __shfl_up(sum, off, 64);
+      sum += lane >= off ? up : 0u;
+    }
+    if (lane == 63) s_wave[wave] = sum;
+    __syncthreads();
+    uint32_t before = 0, total = 0;
+    for (int q = 0; q < 16; ++q) {
+      before += q < wave ? s_wave[q] : 0u;
+      total += s_wave[q];
+    }
+    uint32_t o = at + before + sum - static_cast<uint32_t>(__popc(ok));
+    for (uint32_t q = 0; q < 4; ++q)
+      if (ok >> q & 1u) lists[o++] = v0 + 4 * threadIdx.x + q;
+    at += total;
+    __syncthreads();
+  }
+}
+
+// Candidates of every high (0 where it is not admissible), and whether there are any.
+__global__ __launch_bounds__(256) void split_highs_kernel(GroupView g, int high_rows, int hamming, int low_bits,
+                                                          uint32_t const *__restrict__ starts,
+                                                          uint32_t *__restrict__ sizes, uint32_t *__restrict__ flags) {
+  uint32_t const v = blockIdx.x * 256 + threadIdx.x;
+  int const lx = g.fact_lx;
+  uint32_t const rm = (1u << lx) - 1, pm = (1u << (2 * lx)) - 1;
+  if (v >> (high_rows * lx) != 0) return;
+  uint32_t const top = v >> ((high_rows - 1) * lx);
+  int const w = hamming - __popc(v);
+  uint32_t size = 0;
+  if (w >= 0 && w <= low_bits && least_row(g, top) == top) {
+    bool ok = true;
+    for (int r = 0; r < high_rows - 1 && ok; ++r) ok = least_row(g, v >> (r * lx) & rm) >= top;
+    if (high_rows > 1) {
+      uint32_t const top_pair = v >> ((high_rows - 2) * lx);
+      for (int r = 0; r < high_rows - 1 && ok; ++r) ok = g.line_key[v >> (r * lx) & pm] >= top_pair;
+    }
+    uint32_t const *st = starts + top * (kMaxSplitLow + 2);
+    if (ok) size = st[w + 1] - st[w];
+  }
+  sizes[v] = size;
+  flags[v] = size > 0 ? 1u : 0u;
+}
+
+__global__ __launch_bounds__(256) void split_compact_kernel(uint32_t highs, uint32_t const *__restrict__ sizes,
+                                                            uint64_t const *__restrict__ places,
+                                                            uint64_t const *__restrict__ firsts,
+                                                            uint32_t *__restrict__ out, uint64_t *__restrict__ first,
+                                                            uint64_t count, uint64_t total) {
+  uint32_t const v = blockIdx.x * 256 + threadIdx.x;
+  if (v >= highs) return;
+  if (v == 0) first[count] = total;
+  if (sizes[v] == 0) return;
+  out[places[v]] = v;
+  first[places[v]] = firsts[v];
+}
+
+// The highs of a tile of candidates, in LDS.
+struct SplitTile {
+  int first[kSplitTile + 1]; // first candidate, counted from the tile's (the first may be negative)
+  uint32_t high[kSplitTile + 1];
+  int count;
+};
+
+__device__ __forceinline__ void load_tile(SplitTile &t, SplitView const &s, int64_t base, int candidates) {
+  int64_t lo = 0, hi = s.count - 1; // the last high whose first candidate is <= base
+  while (lo < hi) {
+    int64_t const mid = (lo + hi + 1) / 2;
+    if (static_cast<int64_t>(s.first[mid]) <= base) lo = mid;
+    else hi = mid - 1;
+  }
+  if (threadIdx.x == 0) t.count = 0;
+  __syncthreads();
+  int mine = 0;
+  for (int i = threadIdx.x; i <= kSplitTile && lo + i < s.count; i += 256) {
+    int64_t const f = static_cast<int64_t>(s.first[lo + i]) - base;
+    if (f >= candidates) break;
+    t.first[i] = static_cast<int>(f);
+    t.high[i] = s.highs[lo + i];
+    mine = i + 1;
+  }
+  atomicMax(&t.count, mine);
+  __syncthreads();
+}
+
+__device__ __forceinline__ uint64_t tile_state(SplitTile const &t, SplitView const &s, int lx, int high_rows, int c) {
+  int lo = 0, hi = t.count - 1;
+  while (lo < hi) {
+    int const mid = (lo + hi + 1) >> 1;
+    if (t.first[mid] <= c) lo = mid;
+    else hi = mid - 1;
+  }
+  uint32_t const high = t.high[lo];
+  uint32_t const *st = s.starts + (high >> ((high_rows - 1) * lx)) * (kMaxSplitLow + 2);
+  uint32_t const low = s.lists[st[s.hamming - __popc(high)] + static_cast<uint32_t>(c - t.first[lo])];
+  return static_cast<uint64_t>(high) << (s.low_rows * lx) | low;
+}
+
+template <typename W, int SI>
+__global__ __launch_bounds__(256) void split_count_kernel(GroupView g, SplitView s, uint32_t *__restrict__ bits,
+                                                          uint32_t *__restrict__ counts) {
+  extern __shared__ uint64_t search_lds[];
+  __shared__ SplitTile tile;
+  __shared__ uint64_t s_state[4][128];
+  __shared__ uint16_t s_place[4][128];
+  __shared__ uint32_t s_bits[kSplitTile / 32];
+  LineSearch<W, SI> search;
+  search.stage(g, search_lds);
+  int64_t const base = static_cast<int64_t>(blockIdx.x) * kSplitTile;
+  int const n = static_cast<int>(min(static_cast<int64_t>(kSplitTile), s.total - base));
+  if (threadIdx.x < kSplitTile / 32) s_bits[threadIdx.x] = 0;
+  load_tile(tile, s, base, n); // its barriers cover the staging too
+  int const lx = g.fact_lx, ly = g.fact_ly, top = (ly - 1) * lx, high_rows = ly - s.low_rows;
+  uint32_t const rm = (1u << lx) - 1, pm = (1u << (2 * lx)) - 1;
+  int const lane = static_cast<int>(threadIdx.x) & 63, wave = static_cast<int>(threadIdx.x) >> 6;
+  int queued = 0;
+  auto drain = [&](int m) {
+    __builtin_amdgcn_wave_barrier();
+    if (lane < m) {
+      W const x = static_cast<W>(s_state[wave][lane]);
+      OrbitMinimum<W, SI> const least = search.minimum(g, x);
+      int const stabiliser = least.sum < 0 ? -least.sum : least.sum;
+      if (least.best == x && static_cast<double>(stabiliser) > g.norm_eps) {
+        int const c = s_place[wave][lane];
+        atomicOr(&s_bits[c >> 5], 1u << (c & 31));
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+  };
+  for (int c0 = 64 * wave; c0 < n; c0 += 256) {
+    int const c = c0 + lane;
+    bool on = c < n;
+    uint64_t x = 0;
+    if (on) {
+      x = tile_state(tile, s, lx, high_rows, c);
+      uint32_t const mine = static_cast<uint32_t>(x >> (top - lx));
+      on = x >= s.lower && x <= s.upper;
+#pragma unroll
+      for (int j = 0; j < kMaxLineRows; ++j)
+        if (j < ly) on = on && search.key[search.pair(static_cast<W>(x), j, lx, top, rm, pm)] >= mine;
+    }
+    uint64_t const mask = __ballot(on);
+    if (on) {
+      int const at = queued + __popcll(mask & ((uint64_t{1} << lane) - 1));
+      s_state[wave][at] = x;
+      s_place[wave][at] = static_cast<uint16_t>(c);
+    }
+    queued += __popcll(mask);
+    if (queued >= 64) {
+      drain(64);
+      queued -= 64;
+      if (lane < queued) {
+        s_state[wave][lane] = s_state[wave][64 + lane];
+        s_place[wave][lane] = s_place[wave][64 + lane];
+      }
+    }
+  }
+  if (queued > 0) drain(queued);
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    uint32_t const word = s_bits[threadIdx.x];
+    bits[static_cast<int64_t>(blockIdx.x) * 64 + threadIdx.x] = word;
+    int v = __popc(word);
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    if (threadIdx.x == 0) counts[blockIdx.x] = static_cast<uint32_t>(v);
+  }
+}
+
+__global__ __launch_bounds__(256) void split_write_kernel(GroupView g, SplitView s, uint32_t const *__restrict__ bits,
+                                                          uint32_t const *__restrict__ counts,
+                                                          uint64_t const *__restrict__ offsets,
+                                                          uint64_t *__restrict__ out) {
+  __shared__ SplitTile tile;
+  __shared__ uint32_t s_bits[64], s_before[64];
+  if (counts[blockIdx.x] == 0) return;
+  int64_t const base = static_cast<int64_t>(blockIdx.x) * kSplitTile;
+  int const n = static_cast<int>(min(static_cast<int64_t>(kSplitTile), s.total - base));
+  if (threadIdx.x < 64) {
+    uint32_t const word = bits[static_cast<int64_t>(blockIdx.x) * 64 + threadIdx.x];
+    uint32_t v = static_cast<uint32_t>(__popc(word));
+    for (int off = 1; off < 64; off <<= 1) {
+      uint32_t const up = __shfl_up(v, off, 64);
+      v += static_cast<int>(threadIdx.x) >= off ? up : 0u;
+    }
+    s_bits[threadIdx.x] = word;
+    s_before[threadIdx.x] = v - static_cast<uint32_t>(__popc(word));
+  }
+  load_tile(tile, s, base, n);
+  uint64_t const o = offsets[blockIdx.x];
+  int const lx = g.fact_lx, high_rows = g.fact_ly - s.low_rows;
+  for (int c = threadIdx.x; c < n; c += 256) {
+    uint32_t const word = s_bits[c >> 5];
+    if ((word >> (c & 31) & 1u) == 0) continue;
+    out[o + s_before[c >> 5] + __popc(word & ((1u << (c & 31)) - 1))] = tile_state(tile, s, lx, high_rows, c);
+  }
+}
+static_assert(kSplitTile / 32 == 64, "a tile's acceptance bits are one word per lane");
+
+// ---------------------------------------------------------------------------
 // Driver
 // ---------------------------------------------------------------------------
 
@@ -703,6 +960,97 @@ void release_enumeration_scratch() {
   g_enum_scratch.counts.reset();
   g_enum_scratch.offsets.reset();
   g_enum_scratch.survivors.reset();
+}
+
+// Lower rows of the split (their lists are indexed by top row and weight), 0
+// when the upper rows are too many for a table over their values.
+int split_low_rows(GroupData const &g) {
+  int rows = g.fact_ly / 2;
+  while (rows * g.fact_lx > kMaxSplitLow) --rows;
+  return (g.fact_ly - rows) * g.fact_lx <= kMaxSplitHigh ? rows : 0;
+}
+
+// The split enumeration of [lower, upper]; `out` receives `kept` states.
+bool enumerate_split(GroupData const &g, int hamming, uint64_t lower, uint64_t upper, DeviceArray<uint64_t> &out,
+                     uint64_t &kept) {
+  GroupView const v = g.view();
+  int const lx = g.fact_lx, ly = g.fact_ly, nv = 1 << lx;
+  int const low_rows = split_low_rows(g);
+  int const high_rows = ly - low_rows, low_bits = low_rows * lx;
+  // list lengths by top row and weight: coefficients of (sum over admissible
+  // rows of t^weight)^low_rows
+  constexpr int kWeights = kMaxSplitLow + 2;
+  std::vector<uint32_t> starts(static_cast<size_t>(nv) * kWeights, 0), tops;
+  uint32_t entries = 0;
+  for (int top = 0; top < nv; ++top) {
+    if (g.h_line_least[top] != top) continue;
+    tops.push_back(static_cast<uint32_t>(top));
+    std::vector<uint32_t> count(kWeights, 0);
+    count[0] = 1;
+    for (int r = 0; r < low_rows; ++r) {
+      std::vector<uint32_t> next(kWeights, 0);
+      for (int row = 0; row < nv; ++row)
+        if (g.h_line_least[row] >= top)
+          for (int w = 0; w + __builtin_popcount(row) <= low_bits; ++w) next[w + __builtin_popcount(row)] += count[w];
+      count = next;
+    }
+    for (int w = 0; w <= low_bits + 1; ++w) {
+      starts[static_cast<size_t>(top) * kWeights + w] = entries;
+      if (w <= low_bits) entries += count[w];
+    }
+  }
+  uint32_t const highs = 1u << (high_rows * lx);
+  DeviceArray<uint32_t> d_starts, d_tops, lists, sizes, flags, d_highs;
+  DeviceArray<uint64_t> places, firsts, first;
+  if (!d_starts.upload(starts.data(), starts.size()) || !d_tops.upload(tops.data(), tops.size()) ||
+      !lists.allocate(entries) || !sizes.allocate(highs) || !flags.allocate(highs) || !places.allocate(highs) ||
+      !firsts.allocate(highs))
+    return false;
+  dim3 const grid(static_cast<unsigned>(tops.size()), static_cast<unsigned>(low_bits + 1));
+  split_lists_kernel<<<grid, 1024, 0, stream()>>>(v, low_rows, d_tops.ptr, d_starts.ptr, lists.ptr);
+  LSAMD_HIP(hipGetLastError());
+  split_highs_kernel<<<grid_for(highs, 256), 256, 0, stream()>>>(v, high_rows, hamming, low_bits, d_starts.ptr,
+                                                                 sizes.ptr, flags.ptr);
+  LSAMD_HIP(hipGetLastError());
+  uint64_t count = 0, total = 0;
+  kept = 0;
+  if (!exclusive_scan(flags.ptr, highs, places.ptr, count) || !exclusive_scan(sizes.ptr, highs, firsts.ptr, total))
+    return false;
+  if (total == 0) {
+    out.reset();
+    return true;
+  }
+  if (!d_highs.allocate(count) || !first.allocate(count + 1)) return false;
+  split_compact_kernel<<<grid_for(highs, 256), 256, 0, stream()>>>(highs, sizes.ptr, places.ptr, firsts.ptr,
+                                                                   d_highs.ptr, first.ptr, count, total);
+  LSAMD_HIP(hipGetLastError());
+  int64_t const tiles = (static_cast<int64_t>(total) + kSplitTile - 1) / kSplitTile;
+  DeviceArray<uint32_t> bits, counts;
+  DeviceArray<uint64_t> offsets;
+  if (!bits.allocate(static_cast<size_t>(tiles) * 64) || !counts.allocate(static_cast<size_t>(tiles)) ||
+      !offsets.allocate(static_cast<size_t>(tiles)))
+    return false;
+  SplitView const s{lists.ptr, d_starts.ptr, d_highs.ptr, first.ptr, static_cast<int64_t>(count),
+                    static_cast<int64_t>(total), lower, upper, low_rows, hamming};
+  bool const ok = dispatch_group(g, [&]<typename W, int D, int SI>() -> bool {
+    if constexpr (SI != kFermionic) {
+      split_count_kernel<W, SI><<<static_cast<unsigned>(tiles), 256,
+                                  LineSearch<W, SI>::lds_bytes(g.line_classes, lx, ly, 256), stream()>>>(
+          v, s, bits.ptr, counts.ptr);
+      LSAMD_HIP(hipGetLastError());
+      return true;
+    }
+    return fail("no split enumeration for fermions");
+  });
+  if (!ok || !exclusive_scan(counts.ptr, tiles, offsets.ptr, kept) || !out.allocate(static_cast<size_t>(kept)))
+    return false;
+  if (kept > 0) {
+    split_write_kernel<<<static_cast<unsigned>(tiles), 256, 0, stream()>>>(v, s, bits.ptr, counts.ptr, offsets.ptr,
+                                                                           out.ptr);
+    LSAMD_HIP(hipGetLastError());
+  }
+  LSAMD_HIP(hipStreamSynchronize(stream()));
+  return true;
 }
 
 bool enumerate_states(EnumerationSpec const &spec, uint64_t lower, uint64_t upper,
@@ -786,6 +1134,19 @@ bool enumerate_states(EnumerationSpec const &spec, uint64_t lower, uint64_t uppe
       if (id) q_identity = static_cast<int>(k);
     }
   bool const use_factored = q_identity >= 0;
+  // The split enumeration lists the whole sector's candidates, so it serves
+  // ranges of at least an eighth of the sector (it does about a tenth of the
+  // filter's work: 3.2 against 26.7 ms on 6x6).  It is the faster one at every
+  // size: 0.39 against 0.51 ms on 4x4, 0.62 against 0.91 ms on 5x6.
+  if (use_factored && g.lines() && split_low_rows(g) > 0 &&
+      static_cast<uint64_t>(p.total) >= binomial_host(n, p.hamming) / (spec.spin_inversion != 0 ? 16 : 8)) {
+    uint64_t kept = 0;
+    timer_begin(kTimerEnumerate);
+    if (!enumerate_split(g, p.hamming, lower, hi, out, kept)) return false;
+    timer_end(kTimerEnumerate);
+    count = static_cast<int64_t>(kept);
+    return true;
+  }
   // The element order of the element-by-element filter (kind 0), formed on
   // first use: the factorised filter does not read it.
   DeviceArray<int> d_order;

@@ -424,6 +424,8 @@ bool group_plan_lines(GroupData &g, std::vector<Perm> const &perms) {
     key[p] = static_cast<uint16_t>(least);
     buffer[static_cast<size_t>(p)] = mask;
   }
+  g.h_line_least.resize(static_cast<size_t>(nv));
+  for (int v = 0; v < nv; ++v) g.h_line_least[v] = static_cast<uint8_t>(key[(v << lx) | v] >> lx);
   if (!g.d_line.upload(buffer.data(), buffer.size())) return false;
   g.line_classes = nc;
   return true;

@@ -244,6 +244,7 @@ struct GroupData {
   // of GroupView::line_*.
   int line_classes = 0;
   DeviceArray<uint64_t> d_line;
+  std::vector<uint8_t> h_line_least; // least row an image of a row value can have
   size_t line_off_base = 0, line_off_q = 0, line_off_key = 0, line_off_rot = 0; // bytes
   int run_points = 0;
   bool factored() const { return fact_lx > 0 && fermion_species == 0; }
