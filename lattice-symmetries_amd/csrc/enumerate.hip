@@ -1123,6 +1123,15 @@ bool enumerate_states(EnumerationSpec const &spec, uint64_t lower, uint64_t uppe
   }
 
   GroupData const &g = *spec.group;
+  if (p.hamming == kSpinful && g.species() && g_factored_enumeration.load()) {
+    uint64_t const low = (uint64_t{1} << p.sites) - 1;
+    uint64_t kept = 0;
+    timer_begin(kTimerEnumerate);
+    if (!enumerate_species(g, p.minA, p.maxA, lower >> p.sites & low, upper >> p.sites & low, out, kept)) return false;
+    timer_end(kTimerEnumerate);
+    count = static_cast<int64_t>(kept);
+    return true;
+  }
   GroupView const v = g.view();
   // The factorised filter: fixed Hamming weight, a group of torus
   // translations times point elements with characters +-1, not fermionic.

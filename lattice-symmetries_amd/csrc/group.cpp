@@ -528,7 +528,7 @@ bool group_make_fermionic(GroupData &g, int species) {
   }
   if (!g.d_image.upload(image.data(), image.size())) return false;
   g.fermion_species = species;
-  return true;
+  return species == 1 || group_plan_species(g);
 }
 
 } // namespace lsamd

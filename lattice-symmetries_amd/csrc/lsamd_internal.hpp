@@ -123,9 +123,18 @@ template <typename T> struct DeviceArray {
 };
 
 // What the product has to do with every beta (BatchedOperator.chpl:264-282).
-// The last three are kPermutations through the translation factorisation of
-// the group: state_info_factored, the row-pair search and the run search.
-enum ProjectionKind { kNoProjection = 0, kInversionOnly = 1, kPermutations = 2, kFactored = 3, kLines = 4, kRuns = 5 };
+// kFactored, kLines and kRuns are kPermutations through the translation
+// factorisation of the group (state_info_factored, the row-pair search and the
+// run search), kSpecies through the tables of a spinful fermion group.
+enum ProjectionKind {
+  kNoProjection = 0,
+  kInversionOnly = 1,
+  kPermutations = 2,
+  kFactored = 3,
+  kLines = 4,
+  kRuns = 5,
+  kSpecies = 6
+};
 constexpr bool projects_orbits(int kind) { return kind >= kPermutations; }
 
 // ---------------------------------------------------------------------------
@@ -173,6 +182,15 @@ struct GroupView {
   // Search over the longest runs of zeros (chains with at most kMaxRunPoints
   // point elements).
   int run_points;
+  // Spinful fermions on at most 16 sites (species_entry = null: none; see
+  // species.hip): per state of one species the least image | number of
+  // elements reaching it << 16 | their place in species_list << 32, the sign
+  // of every element on every such state (bits), and the elements' ranks in
+  // the state_info reduction.
+  uint64_t const *species_entry;
+  uint16_t const *species_list;
+  uint32_t const *species_sign;
+  int32_t const *species_rank;
 };
 
 // Sorted representatives plus a prefix table over their top bits:
@@ -247,6 +265,12 @@ struct GroupData {
   std::vector<uint8_t> h_line_least; // least row an image of a row value can have
   size_t line_off_base = 0, line_off_q = 0, line_off_key = 0, line_off_rot = 0; // bytes
   int run_points = 0;
+  // Tables of the spinful search (group_plan_species).
+  DeviceArray<uint64_t> d_species_entry;
+  DeviceArray<uint16_t> d_species_list;
+  DeviceArray<uint32_t> d_species_sign;
+  DeviceArray<int32_t> d_species_rank;
+  bool species() const { return fermion_species == 2 && d_species_entry.ptr != nullptr; }
   bool factored() const { return fact_lx > 0 && fermion_species == 0; }
   bool lines() const { return factored() && line_classes > 0; }
   bool runs() const { return factored() && run_points > 0; }
@@ -258,7 +282,8 @@ struct GroupData {
                      d_fact_key.ptr, fact_m1, fact_m2, fact_uniform ? 1 : 0, line_classes,
                      reinterpret_cast<uint16_t const *>(line + line_off_key), d_line.ptr,
                      reinterpret_cast<uint64_t const *>(line + line_off_base), line + line_off_rot,
-                     reinterpret_cast<int32_t const *>(line + line_off_q), run_points};
+                     reinterpret_cast<int32_t const *>(line + line_off_q), run_points,
+                     d_species_entry.ptr, d_species_list.ptr, d_species_sign.ptr, d_species_rank.ptr};
   }
 };
 
@@ -278,6 +303,18 @@ constexpr int kMaxRunPoints = 2;
 // fall into classes under row and column reflections, and the run search of a
 // chain (line_classes = run_points = 0 where they do not apply).
 bool group_plan_lines(GroupData &g, std::vector<std::vector<int32_t>> const &perms);
+
+// Tables of the spinful search (species.hip) for a fermionic group of two
+// species on at most kMaxSpeciesSites sites whose characters have real part
+// +-1 and whose networks fit LDS; leaves species() false otherwise.
+constexpr int kMaxSpeciesSites = 16;
+constexpr size_t kMaxSpeciesLds = 24 << 10;
+size_t species_lds_bytes(GroupData const &g);
+bool group_plan_species(GroupData &g);
+// Representatives of a spinful basis with those tables: products of up states
+// in [min_up, max_up] and down states in [min_down, max_down].
+bool enumerate_species(GroupData const &g, uint64_t min_up, uint64_t max_up, uint64_t min_down, uint64_t max_down,
+                       DeviceArray<uint64_t> &out, uint64_t &kept);
 
 // Marks a group as fermionic (species 1 or 2) and uploads the orbital
 // images; spin inversion must be off.
@@ -332,6 +369,9 @@ void release_enumeration_scratch();
 bool enumerate_states(EnumerationSpec const &spec, uint64_t lower,
                       uint64_t upper, DeviceArray<uint64_t> &out,
                       int64_t &count, int64_t &candidates);
+
+// offsets[0 .. n): exclusive sums of counts; `total` the whole sum.
+bool exclusive_scan(uint32_t const *d_counts, int64_t n, uint64_t *d_offsets, uint64_t &total);
 
 // Orbit kernels on device arrays (orbit.hip).
 bool launch_state_info(GroupData const &g, int64_t count, uint64_t const *d_x,

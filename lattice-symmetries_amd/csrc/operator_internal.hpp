@@ -113,7 +113,6 @@ bool apply_off_diag_device(Terms const &t, int64_t count, uint64_t const *d_alph
                            DeviceArray<double> &coeffs, DeviceArray<int64_t> &offsets,
                            int64_t &total);
 
-bool exclusive_scan(uint32_t const *d_counts, int64_t n, uint64_t *d_offsets, uint64_t &total);
 
 // Thick-restart block Lanczos on FP64 row-major [rows][block] blocks over
 // independent segments of rows (block_krylov.hip).

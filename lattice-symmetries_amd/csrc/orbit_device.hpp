@@ -641,6 +641,78 @@ template <typename W, int D, int SI> struct RunSearch {
   }
 };
 
+// Spinful search (GroupView::species_*).  Every element acts alike on the two
+// species, and the down species holds the high bits, so the least image has
+// the least image of the down state, reached by a few elements (one, unless
+// the down state has a stabiliser) that a table lists; only their images of
+// the up state are formed.  Signs come from a bit table per species: the
+// species do not pass each other.  On the 4x4 Hubbard sector (128 elements)
+// this replaces 128 networks of 9 stages per state: the complex on-the-fly
+// product takes 1.7 ms against 11.8 ms, now bound by its atomics (42 G/s), and
+// the norms 0.02 ms.
+template <typename W, int D> struct SpeciesSearch {
+  W *masks; // LDS: the networks, element-major
+  double norm_1;
+
+  // Every thread of the workgroup must call it; a barrier follows.
+  __device__ __forceinline__ void stage(GroupView const &g, void *smem) {
+    masks = static_cast<W *>(smem);
+    int const count = g.size * g.depth;
+    for (int i = threadIdx.x; i < count; i += blockDim.x) masks[i] = static_cast<W>(g.masks[i]);
+    norm_1 = sqrt(1.0 / static_cast<double>(g.size));
+  }
+
+  __device__ __forceinline__ bool odd(GroupView const &g, int e, uint32_t s, int words) const {
+    return (g.species_sign[static_cast<size_t>(e) * words + (s >> 5)] >> (s & 31) & 1u) != 0;
+  }
+
+  __device__ __forceinline__ W up_image(GroupView const &g, int e, W up) const {
+    return benes_apply_ptr<W, D>(masks + static_cast<size_t>(e) * g.depth, up, g.shifts, g.depth);
+  }
+
+  __device__ __forceinline__ StateInfo info(GroupView const &g, uint64_t x) const {
+    int const sites = g.nbits / 2, words = ((1 << sites) + 31) / 32;
+    uint32_t const mask = (1u << sites) - 1;
+    uint32_t const up = static_cast<uint32_t>(x) & mask, down = static_cast<uint32_t>(x >> sites) & mask;
+    uint64_t const entry = g.species_entry[down];
+    int const count = static_cast<int>(entry >> 16 & 0xffffu);
+    uint16_t const *list = g.species_list + (entry >> 32);
+    W best = ~W{0};
+    int element = 0, sum = 0;
+    double sign = 1.0;
+    for (int i = 0; i < count; ++i) {
+      int const e = list[i];
+      W const y = up_image(g, e, static_cast<W>(up));
+      if (y > best) continue;
+      bool const minus = odd(g, e, up, words) != odd(g, e, down, words);
+      int const term = (g.eig_re[e] < 0.0) != minus ? -1 : 1;
+      if (y < best || g.species_rank[e] < g.species_rank[element]) { // of equal images the lowest rank
+        element = e;
+        sign = minus ? -1.0 : 1.0;
+      }
+      sum = y < best ? term : sum + term;
+      best = y;
+    }
+    StateInfo out;
+    out.rep = (entry & 0xffffu) << sites | static_cast<uint64_t>(best);
+    if (out.rep == x) {
+      out.c_re = 1.0;
+      out.c_im = 0.0;
+    } else {
+      out.c_re = g.eig_re[element] * sign;
+      out.c_im = g.eig_im[element] * sign;
+    }
+    int const n = sum < 0 ? -sum : sum;
+    if (n == 1 && g.norm_eps <= 0.0) {
+      out.norm = norm_1;
+    } else {
+      double const nn = static_cast<double>(n);
+      out.norm = (g.norm_eps > 0.0 && !(nn > g.norm_eps)) ? 0.0 : sqrt(nn / static_cast<double>(g.size));
+    }
+    return out;
+  }
+};
+
 // state_info of one kernel kind, with its tables staged in LDS: static shared
 // memory for kFactored, dynamic at `smem` (search_lds_bytes) for the others.
 template <typename W, int D, int SI, int KIND> struct OrbitSearch {
@@ -665,10 +737,17 @@ template <typename W, int D, int SI> struct OrbitSearch<W, D, SI, kLines> : Line
   }
 };
 template <typename W, int D, int SI> struct OrbitSearch<W, D, SI, kRuns> : RunSearch<W, D, SI> {};
+template <typename W, int D, int SI> struct OrbitSearch<W, D, SI, kSpecies> : SpeciesSearch<W, D> {
+  __device__ __forceinline__ void stage(GroupView const &g, void *smem) {
+    SpeciesSearch<W, D>::stage(g, smem);
+    __syncthreads();
+  }
+};
 
 template <typename W, int D, int SI, int KIND> size_t search_lds_bytes(GroupData const *g, int threads) {
   if constexpr (KIND == kLines) return LineSearch<W, SI>::lds_bytes(g->line_classes, g->fact_lx, g->fact_ly, threads);
   if constexpr (KIND == kRuns) return RunSearch<W, D, SI>::lds_bytes(threads);
+  if constexpr (KIND == kSpecies) return species_lds_bytes(*g);
   return 0;
 }
 
@@ -789,8 +868,8 @@ template <typename F> bool dispatch_group(GroupData const &g, F &&f) {
   return by_si.template operator()<uint64_t, 0>();
 }
 
-// Dispatch on (W, D, SI, KIND) of the orbit search of a group: the row-pair or
-// run search where the group has one and its tables fit LDS beside the `lds`
+// Dispatch on (W, D, SI, KIND) of the orbit search of a group: the row-pair,
+// run or spinful search where the group has one and its tables fit LDS beside the `lds`
 // bytes the kernel needs for itself, else the factorised search where it
 // factors (`factored` allowed), else element by element.  The row-pair search
 // applies no networks, so its kernels do not depend on the depth.
@@ -804,6 +883,9 @@ template <typename F> bool dispatch_search(GroupData const &g, bool factored, si
       if (factored && g.runs() && lds + search_lds_bytes<W, D, SI, kRuns>(&g, 256) <= kSearchLds)
         return f.template operator()<W, D, SI, kRuns>();
       if (factored && g.factored()) return f.template operator()<W, D, SI, kFactored>();
+    } else {
+      if (factored && g.species() && lds + species_lds_bytes(g) <= kSearchLds)
+        return f.template operator()<W, D, SI, kSpecies>();
     }
     return f.template operator()<W, D, SI, kPermutations>();
   });
