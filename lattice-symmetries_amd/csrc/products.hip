@@ -58,9 +58,9 @@ template <typename F> bool dispatch_k(int k, F &&f) {
 // The schedule of a block product, by the bytes of x it gathers per stored
 // entry: up to 16 B (FP32 blocks of 1, 2, 4; FP64 blocks of 1, 2) the one
 // tuned on the FP64 vector (8 B), above that the one tuned on the FP32 block
-// of 8 (32 B).  On 6x6 the die-aware full grid that suits the narrow
-// gathers takes the FP32 block of 2 from 6.85 to 6.01 ms, while the block
-// of 8 is fastest on the plain grid.
+// of 8 (32 B).  On 6x6 both are fastest with 16 lanes on the die-aware full
+// grid (the FP32 block of 2 5.6 against 6.8 ms on the plain grid, the block of
+// 8 9.2 against 10.2 ms); where x stays on chip the widths may differ.
 struct Schedule {
   int lanes, flags;
 };

@@ -102,27 +102,38 @@ __global__ __launch_bounds__(kThreads) void sector_spmv_kernel(int64_t n, int64_
     t_end = tiles;
     t_step = gridDim.x;
   }
+  // As in csr_block_rows, several lanes share an entry: each takes kPart
+  // columns, 16 bytes of the real and of the imaginary parts where K allows.
+  // 52 sectors of the 26-site chain, 8 columns: FP32 2.84 -> 2.43 ms, FP64 6.94
+  // -> 3.88 ms; two or four entries in flight per lane gain nothing more (2.52,
+  // 2.66 ms: rows of 27 entries leave remainders).  Bound by the L2 misses of
+  // the x rows and the 12 (20) bytes of column and value per entry.
+  constexpr int kWant = static_cast<int>(sizeof(T)) * K / 16;
+  constexpr int kShare = kWant < 1 ? 1 : (kWant < LPR ? kWant : LPR);
+  constexpr int kPart = K / kShare;
+  constexpr int kStep = LPR / kShare;
   int const sub = static_cast<int>(threadIdx.x) % LPR;
   int const r_in = static_cast<int>(threadIdx.x) / LPR;
   T2 const *__restrict__ v2 = reinterpret_cast<T2 const *>(vals);
+  T const *__restrict__ xp = x + sub % kShare * kPart;
   for (; t < t_end; t += t_step) {
     int64_t const row = t * kRows + r_in;
-    T re[K], im[K];
+    T re[kPart], im[kPart];
 #pragma unroll
-    for (int q = 0; q < K; ++q) re[q] = im[q] = T(0);
+    for (int q = 0; q < kPart; ++q) re[q] = im[q] = T(0);
     if (row < n) {
       int64_t const b = rp[row], e = rp[row + 1];
-      for (int64_t k = b + sub; k < e; k += LPR) {
+      for (int64_t k = b + sub / kShare; k < e; k += kStep) {
         T2 const v = v2[k];
-        T const *__restrict__ xr = x + static_cast<size_t>(cols[k]) * (2 * K);
-        T xre[K], xim[K];
+        T const *__restrict__ xr = xp + static_cast<size_t>(cols[k]) * (2 * K);
+        T xre[kPart], xim[kPart];
 #pragma unroll
-        for (int q = 0; q < K; ++q) {
+        for (int q = 0; q < kPart; ++q) {
           xre[q] = xr[q];
           xim[q] = xr[K + q];
         }
 #pragma unroll
-        for (int q = 0; q < K; ++q) {
+        for (int q = 0; q < kPart; ++q) {
           re[q] = fma(v.x, xre[q], re[q]);
           re[q] = fma(-v.y, xim[q], re[q]);
           im[q] = fma(v.y, xre[q], im[q]);
@@ -131,19 +142,19 @@ __global__ __launch_bounds__(kThreads) void sector_spmv_kernel(int64_t n, int64_
       }
     }
 #pragma unroll
-    for (int q = 0; q < K; ++q) {
+    for (int q = 0; q < kPart; ++q) {
 #pragma unroll
-      for (int off = LPR / 2; off > 0; off >>= 1) {
+      for (int off = LPR / 2; off >= kShare; off >>= 1) {
         re[q] += __shfl_xor(re[q], off, LPR);
         im[q] += __shfl_xor(im[q], off, LPR);
       }
     }
-    if (row < n && sub == 0) {
+    if (row < n && sub < kShare) {
       T const d = diag[row];
-      T const *__restrict__ xi = x + static_cast<size_t>(row) * (2 * K);
-      TO *__restrict__ yi = y + static_cast<size_t>(row) * (2 * K);
+      T const *__restrict__ xi = xp + static_cast<size_t>(row) * (2 * K);
+      TO *__restrict__ yi = y + static_cast<size_t>(row) * (2 * K) + sub * kPart;
 #pragma unroll
-      for (int q = 0; q < K; ++q) {
+      for (int q = 0; q < kPart; ++q) {
         yi[q] = static_cast<TO>(fma(d, xi[q], re[q]));
         yi[K + q] = static_cast<TO>(fma(d, xi[K + q], im[q]));
       }

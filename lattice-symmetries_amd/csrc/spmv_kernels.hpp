@@ -168,61 +168,71 @@ __global__ __launch_bounds__(256) void csr_f64_wide_kernel(int64_t n, int64_t co
 }
 
 // y[row][q] = diag[row] x[row][q] + sum of the row's entries v x[col][q] for
-// K right-hand sides stored [rows][K], summed in T.
+// K right-hand sides stored [rows][K], summed in T.  A row of x of more than
+// 16 bytes is read by several lanes, 16 bytes each, so that one load
+// instruction takes the whole row from its cache line: with a lane reading all
+// of it, every further 16 bytes cost another look-up of the line.  On 6x6 the
+// FP32 block of 8 takes 9.2 against 10.1 ms, the FP64 blocks of 4 and 8 9.2
+// and 12.7 against 10.1 and 15.9 ms (die-aware full grid, which one lane to a
+// row of x did not favour); four entries in flight instead of two take 0.1 to
+// 0.2 ms off every width.  Bound by the x rows that miss L2.
 template <int K, int LPR, typename T, typename TO, bool DIE, typename Entries>
 __device__ __forceinline__ void csr_block_rows(int64_t n, int64_t const *__restrict__ rp, Entries const &ent,
                                                T const *__restrict__ diag, T const *__restrict__ x,
                                                TO *__restrict__ y) {
   constexpr int kRows = 256 / LPR;
+  constexpr int kWant = static_cast<int>(sizeof(T)) * K / 16;
+  constexpr int kShare = kWant < 1 ? 1 : (kWant < LPR ? kWant : LPR); // lanes of an entry
+  constexpr int kPart = K / kShare;                                   // values of a lane
+  constexpr int kStep = LPR / kShare;                                 // entries of a row at a time
+  constexpr int kAhead = 4;
   int64_t const tiles = (n + kRows - 1) / kRows;
   int64_t t, t_end, t_step;
   tile_range<DIE>(tiles, t, t_end, t_step);
-  int const sub = static_cast<int>(threadIdx.x) % LPR;
+  int const sub = static_cast<int>(threadIdx.x) % LPR, first = sub / kShare;
+  T const *__restrict__ xp = x + sub % kShare * kPart;
   for (; t < t_end; t += t_step) {
     int64_t const row = t * kRows + static_cast<int>(threadIdx.x) / LPR;
-    T acc[K];
+    T acc[kPart];
 #pragma unroll
-    for (int q = 0; q < K; ++q) acc[q] = T(0);
+    for (int q = 0; q < kPart; ++q) acc[q] = T(0);
     if (row < n) {
       int64_t const b = rp[row], e = rp[row + 1];
-      int64_t k = b + sub;
-      // two entries per step, their gathers in flight together, summed in order
-      for (; k + LPR < e; k += 2 * LPR) {
-        uint32_t c0, c1;
-        T v0, v1;
-        ent(k, c0, v0);
-        ent(k + LPR, c1, v1);
-        T const *x0 = x + static_cast<size_t>(c0) * K;
-        T const *x1 = x + static_cast<size_t>(c1) * K;
-        T a0[K], a1[K];
+      int64_t k = b + first;
+      // kAhead entries per step, their gathers in flight together, summed in order
+      for (; k + (kAhead - 1) * kStep < e; k += kAhead * kStep) {
+        uint32_t c[kAhead];
+        T v[kAhead], a[kAhead][kPart];
 #pragma unroll
-        for (int q = 0; q < K; ++q) {
-          a0[q] = x0[q];
-          a1[q] = x1[q];
-        }
+        for (int u = 0; u < kAhead; ++u) ent(k + u * kStep, c[u], v[u]);
 #pragma unroll
-        for (int q = 0; q < K; ++q) acc[q] = fma(v0, a0[q], acc[q]);
+        for (int u = 0; u < kAhead; ++u)
 #pragma unroll
-        for (int q = 0; q < K; ++q) acc[q] = fma(v1, a1[q], acc[q]);
+          for (int q = 0; q < kPart; ++q) a[u][q] = xp[static_cast<size_t>(c[u]) * K + q];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+          for (int q = 0; q < kPart; ++q) acc[q] = fma(v[u], a[u][q], acc[q]);
       }
-      for (; k < e; k += LPR) {
+      for (; k < e; k += kStep) {
         uint32_t col;
         T v;
         ent(k, col, v);
-        T const *xr = x + static_cast<size_t>(col) * K;
+        T const *xr = xp + static_cast<size_t>(col) * K;
 #pragma unroll
-        for (int q = 0; q < K; ++q) acc[q] = fma(v, xr[q], acc[q]);
+        for (int q = 0; q < kPart; ++q) acc[q] = fma(v, xr[q], acc[q]);
       }
     }
 #pragma unroll
-    for (int q = 0; q < K; ++q)
+    for (int q = 0; q < kPart; ++q)
 #pragma unroll
-      for (int off = LPR / 2; off > 0; off >>= 1) acc[q] += __shfl_xor(acc[q], off, LPR);
-    if (row < n && sub == 0) {
+      for (int off = LPR / 2; off >= kShare; off >>= 1) acc[q] += __shfl_xor(acc[q], off, LPR);
+    if (row < n && sub < kShare) {
       T const d = diag[row];
+      T const *xr = xp + static_cast<size_t>(row) * K;
+      TO *yr = y + static_cast<size_t>(row) * K + sub * kPart;
 #pragma unroll
-      for (int q = 0; q < K; ++q)
-        y[static_cast<size_t>(row) * K + q] = static_cast<TO>(d * x[static_cast<size_t>(row) * K + q] + acc[q]);
+      for (int q = 0; q < kPart; ++q) yr[q] = static_cast<TO>(d * xr[q] + acc[q]);
     }
   }
 }
