@@ -1,4 +1,4 @@
-// operator.hip -- term application, fused product, CSR cache and SpMV.
+// operator.hip -- term application, fused product and the CSR cache's build.
 //
 // The reference applies H in push form: every representative alpha_i emits
 // (beta, c) pairs, c is rescaled by chi_beta n_beta / n_alpha after
@@ -7,14 +7,16 @@
 // chapel/src/DistributedMatrixVector.chpl:91-143).  The engine computes the
 // same matrix M, M[index(rep beta), i] = C, for every operator, Hermitian or
 // not:
-// - the fused on-the-fly product is push form too: one lane per alpha_i,
-//   the diagonal pass first, then atomic adds of Re(c) (or c x_i for complex
-//   vectors) into y;
-// - the CSR build emits the pairs of each alpha_i as a source row, then
-//   transposes them on the device (count -> scan -> scatter -> per-row sort),
-//   so that row j of the cached matrix holds every (i, C) with target j, in
-//   ascending i.  Products then gather x along a row and write y once,
-//   without atomics, and every build stores the same bits.
+// - the fused on-the-fly product is push form too: one lane per (alpha_i,
+//   term) pair, the diagonal pass first, then atomic adds of Re(c) (or c x_i
+//   for complex vectors) into y;
+// - the CSR build emits the pairs of every alpha_i and turns them into target
+//   rows on the device: with a value table the fill pass counts and places the
+//   targets and one scatter writes the final words; otherwise the entries are
+//   counted, scattered and sorted by key.  Row j of the cached matrix holds
+//   every (i, C) with target j, in ascending i.  Products then gather x along
+//   a row and write y once, without atomics, and every build stores the same
+//   bits.
 #include <algorithm>
 #include <cstring>
 
@@ -1127,6 +1129,8 @@ __global__ __launch_bounds__(256) void pack_wide_kernel(double const *__restrict
   vidx[k] = static_cast<uint16_t>(lo);
 }
 
+// For matrices that build_table_csr leaves to the general build although
+// their values are few (a target row of more than 4095 entries).
 // Replaces the value arrays of a real CSR by a value table: packed into the
 // column words when it has at most 256 distinct values and fewer than 2^24
 // rows, else a wide table with 16-bit indices when it has at most
