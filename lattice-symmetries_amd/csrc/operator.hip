@@ -1130,7 +1130,7 @@ __global__ __launch_bounds__(256) void pack_wide_kernel(double const *__restrict
 }
 
 // For matrices that build_table_csr leaves to the general build although
-// their values are few (a target row of more than 4095 entries).
+// their values are few (a target row of more than 4096 entries).
 // Replaces the value arrays of a real CSR by a value table: packed into the
 // column words when it has at most 256 distinct values and fewer than 2^24
 // rows, else a wide table with 16-bit indices when it has at most
@@ -1268,7 +1268,7 @@ __global__ __launch_bounds__(256) void split_wide_keys_kernel(int64_t nnz, uint6
 // 8-byte keys through atomic cursors (42 ms), their LDS sort (24 ms), a gather
 // of the values in target order (23 ms), the distinct-value pass and the
 // packing (11 ms), and the temporaries shrink from 28 to 14 GB.  `done` stays false when the matrix has too many values, a
-// target row of more than 4095 entries, or no entries: then the general
+// target row of more than 4096 entries, or no entries: then the general
 // build runs.
 bool build_table_csr(OperatorCore &op, int64_t up, int64_t const *row_ptr, bool &done) {
   done = false;

@@ -24,6 +24,13 @@ CASES = [
     (6, 6, 7, None, "full", [3, 3, 1, 1, 2]),
     (6, 6, 6, None, "c4", None),
     (2, 8, 8, 1, "full", None),
+    (2, 2, 2, 1, "full", None),
+    (3, 3, 1, None, "full", None),
+    (4, 4, 0, None, "full", None),
+    (4, 4, 16, None, "c4", None),
+    (6, 2, 6, -1, "full", None),
+    (6, 6, 1, None, "full", None),
+    (6, 6, 35, None, "none", None),
 ]
 
 
