@@ -590,7 +590,13 @@ __global__ __launch_bounds__(kPairThreads) void csr_fill_kernel(GroupView g, OpV
   __shared__ WaveRows waves[kPairThreads / 64];
   __shared__ uint32_t s_kept[OUT == kFillTable ? 1 : kPairThreads];
   if constexpr (OUT == kFillTable) {
-    if (*static_cast<int volatile *>(hash.overflow) != 0) return; // the pass is repeated without the table
+    // The pass is repeated without the table.  Other workgroups raise the flag
+    // at any time, so one thread reads it for all: the staging below needs
+    // every thread of a workgroup that goes on.
+    __shared__ int s_stop;
+    if (threadIdx.x == 0) s_stop = *static_cast<int volatile *>(hash.overflow);
+    __syncthreads();
+    if (s_stop != 0) return;
   }
   int const T = op.off.count;
   TermsLds const l = stage_terms(op.off, smem);
@@ -1296,8 +1302,13 @@ bool build_table_csr(OperatorCore &op, int64_t up, int64_t const *row_ptr, bool 
   LSAMD_HIP(hipMemcpyAsync(h.data(), slots.ptr, sizeof(unsigned long long) * kValueSlots, hipMemcpyDeviceToHost,
                            stream()));
   LSAMD_HIP(hipMemcpyAsync(h_flags, flags.ptr, sizeof(h_flags), hipMemcpyDeviceToHost, stream()));
-  if (!check_error(op)) return false; // waits for the copies
-  if (h_flags[1] != 0 || h_flags[0] == 0) return true;
+  LSAMD_HIP(hipStreamSynchronize(stream()));
+  if (h_flags[1] != 0) { // the general build goes over every pair again and reports what it finds
+    LSAMD_HIP(hipMemsetAsync(op.d_err.ptr, 0, sizeof(int), stream()));
+    return true;
+  }
+  if (!check_error(op)) return false;
+  if (h_flags[0] == 0) return true;
   std::vector<std::pair<double, int>> values;
   for (int q = 0; q < kValueSlots; ++q)
     if (h[q] != kEmptySlot) {

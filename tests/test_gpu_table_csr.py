@@ -79,3 +79,77 @@ def test_table_build_equals_the_general_build(engine, name):
     scale = max(np.abs(a).max(initial=0) for a in plain.csr_arrays()[2:]) * np.abs(x).max()
     bound = np.finfo(float).eps * longest ** 2 * scale
     assert np.abs(table.matvec(x, "otf") - plain.matvec(x, "csr")).max() <= bound
+
+
+def projected_flips(count):
+    """`count` distinct values: term k flips bits above the low six where these
+    hold k mod 64, so a row has count / 64 entries."""
+    out = {}
+    for k in range(count):
+        low = k % 64
+        x = (k // 64 + 1) << 6
+        out[(63, low, low, x, 0)] = 1.0 + k / 4096.0
+    return Expr(out)
+
+
+def conditional_hops(n):
+    """Hops i -> j that ask for a third site up or down, each with a coupling of its own."""
+    out = {}
+    for i in range(n):
+        for j in range(n):
+            if i == j:
+                continue
+            k = next(q % n for q in range(max(i, j) + 1, max(i, j) + 4) if q % n not in (i, j))
+            for up in (0, 1):
+                m, r = 1 << i | 1 << j | 1 << k, 1 << i | up << k
+                out[(m, r ^ 1 << i ^ 1 << j, r, 1 << i | 1 << j, 0)] = 1.0 + len(out) / 4096.0
+    return Expr(out)
+
+
+# More workgroups than fit the chip at once, so that some start before and some
+# after the value hash is found full: without a group on both sides of its
+# limit, and with the row-pair search staged beside the terms (576 elements;
+# 2520 couplings times at least two norm ratios).
+FULL_HASH = {
+    "values4096": (lambda: (basis(16), projected_flips(4096)), 4096),
+    "values4097": (lambda: (basis(16), projected_flips(4097)), None),
+    "torus6x6": (lambda: (torus_basis(6, 7), conditional_hops(36)), None),
+}
+
+
+def torus_basis(side, weight):
+    S = lsamd.Symmetries([lsamd.Symmetry(g, 0) for g in models.square_generators(side)])
+    b = lsamd.DeviceBasis(side * side, weight, None, S)
+    b.build()
+    return b
+
+
+@pytest.mark.parametrize("name", FULL_HASH)
+def test_a_full_value_hash_leaves_the_general_build(engine, name):
+    make, distinct = FULL_HASH[name]
+    b, expr = make()
+    print(name, b.number_states, flush=True)
+    plain = lsamd.DeviceOperator(b, expr)
+    plain.set_csr_packing(False)
+    nnz = plain.build_csr(64)
+    want = plain.csr_arrays()
+    for _ in range(3):
+        op = lsamd.DeviceOperator(b, expr)
+        assert op.build_csr(64) == nnz
+        info = op.csr_info
+        assert not info["packed"]
+        assert (info["wide"], info["table_size"]) == ((True, distinct) if distinct else (False, 0))
+        for got, ref in zip(op.csr_arrays(), want):
+            assert np.array_equal(got, ref)
+    if distinct is None:
+        assert np.unique(want[2]).size > 4096
+
+
+def test_a_full_value_hash_still_reports_states_outside_the_basis(engine):
+    b = basis(16, 8)
+    op = lsamd.DeviceOperator(b, projected_flips(4097))
+    for _ in range(2):
+        with pytest.raises(lsamd.EngineError, match="invalid index"):
+            op.build_csr(64)
+    good = lsamd.DeviceOperator(b, models.heisenberg_chain(16))
+    assert good.build_csr(64) > 0
