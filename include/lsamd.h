@@ -203,6 +203,11 @@ void ls_amd_clear_error(void);
 /* Device memory for callers without their own allocator. */
 void *ls_amd_device_malloc(size_t bytes);
 void ls_amd_device_free(void *ptr);
+/* Gives the device blocks that the library keeps for its own later
+   allocations (at most LSAMD_POOL_BYTES) back to the driver, for callers with
+   another allocator that needs them; cached operators stay.  Returns the bytes
+   given back. */
+int64_t ls_amd_device_trim(void);
 int ls_amd_memcpy_h2d(void *dst, void const *src, size_t bytes);
 int ls_amd_memcpy_d2h(void *dst, void const *src, size_t bytes);
 int ls_amd_synchronize(void);

@@ -178,9 +178,11 @@ void pool_release(void *ptr) {
   p.shrink(p.capacity);
 }
 
-void pool_trim() {
+size_t pool_trim() {
   std::lock_guard<std::mutex> lock(pool().mutex);
+  size_t const before = pool().cached;
   pool().shrink(0);
+  return before - pool().cached;
 }
 
 size_t pool_cached_bytes() {
@@ -201,12 +203,16 @@ extern "C" void ls_amd_clear_error(void) { g_last_error.clear(); }
 extern "C" void *ls_amd_device_malloc(size_t bytes) {
   if (!ensure_device()) return nullptr;
   void *p = nullptr;
-  if (hipMalloc(&p, bytes == 0 ? 1 : bytes) != hipSuccess) {
-    set_last_error("hipMalloc failed");
-    return nullptr;
-  }
-  return p;
+  if (hipMalloc(&p, bytes == 0 ? 1 : bytes) == hipSuccess) return p;
+  (void)hipGetLastError();
+  pool_trim(); // the blocks kept for reuse may be what is missing
+  if (hipMalloc(&p, bytes == 0 ? 1 : bytes) == hipSuccess) return p;
+  (void)hipGetLastError();
+  set_last_error("hipMalloc failed");
+  return nullptr;
 }
+
+extern "C" int64_t ls_amd_device_trim(void) { return static_cast<int64_t>(pool_trim()); }
 
 extern "C" void ls_amd_device_free(void *ptr) {
   if (ptr != nullptr) (void)hipFree(ptr);

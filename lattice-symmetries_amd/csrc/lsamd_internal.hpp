@@ -73,10 +73,10 @@ void timer_end(int family);
 // Device memory for DeviceArray.  Freed blocks are kept for later allocations
 // of nearly their size (device.cpp), up to pool_capacity() bytes together;
 // the least recently freed go back to the driver first, and all of them when
-// an allocation fails and on ls_chpl_finalize.
+// an allocation fails, on ls_amd_device_trim and on ls_chpl_finalize.
 void *pool_allocate(size_t bytes); // null when the device is out of memory
 void pool_release(void *ptr);
-void pool_trim();
+size_t pool_trim(); // bytes given back
 size_t pool_cached_bytes();
 
 // RAII device buffer.

@@ -39,11 +39,18 @@ __all__ = [
     "Model",
     "Term",
     "device_available",
+    "device_trim",
 ]
 
 
 def device_available() -> bool:
     return load().ls_amd_device_available() == 0
+
+
+def device_trim() -> int:
+    """Gives the device memory that the engine keeps for reuse back to the
+    driver (for torch or another allocator); returns the bytes."""
+    return int(load().ls_amd_device_trim())
 
 
 def _u64ptr(a: np.ndarray):

@@ -200,6 +200,7 @@ SIGNATURES = {
     "ls_amd_last_error": (C.c_char_p, []),
     "ls_amd_clear_error": (None, []),
     "ls_amd_device_malloc": (_P, [C.c_size_t]),
+    "ls_amd_device_trim": (C.c_int64, []),
     "ls_amd_device_free": (None, [_P]),
     "ls_amd_memcpy_h2d": (C.c_int, [_P, _P, C.c_size_t]),
     "ls_amd_memcpy_d2h": (C.c_int, [_P, _P, C.c_size_t]),

@@ -54,3 +54,28 @@ def test_finalize_gives_the_memory_back(engine):
     del operator, basis
     lib.ls_chpl_finalize()
     assert torch.cuda.mem_get_info()[0] >= before - (64 << 20)
+
+
+def keep_blocks():
+    """Blocks of a released operator and basis stay with the engine."""
+    lsamd.device_trim()
+    free = torch.cuda.mem_get_info()[0]
+    product(24, 1)
+    return free
+
+
+def test_trim_gives_the_memory_back(engine):
+    free = keep_blocks()
+    assert torch.cuda.mem_get_info()[0] < free - (8 << 20)
+    assert lsamd.device_trim() > 8 << 20
+    assert torch.cuda.mem_get_info()[0] >= free - (8 << 20)
+    assert lsamd.device_trim() == 0
+
+
+def test_a_failing_allocation_empties_the_pool_first(engine):
+    free = keep_blocks()
+    assert torch.cuda.mem_get_info()[0] < free - (8 << 20)
+    with pytest.raises(lsamd.EngineError, match="allocation failed"):
+        lsamd.DeviceArray(1 << 50)  # more than any device has
+    assert torch.cuda.mem_get_info()[0] >= free - (8 << 20)
+    assert np.isfinite(product(16, 1)).all()  # and the engine goes on
