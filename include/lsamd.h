@@ -380,8 +380,9 @@ int ls_amd_operator_is_hermitian(ls_amd_operator *op, int mode);
 int ls_amd_operator_schedule(ls_amd_operator const *op, int *out);
 /* Process-wide: whether basis builds may use the translation-factorised
    filter for groups of torus translations times point elements with
-   characters +-1 (1, the default) or always test element by element (0).
-   Both give the same representatives. */
+   characters +-1 (1, the default) or always test element by element (0).  2:
+   as 1, with the upper and lower rows of a torus listed apart also for sectors
+   so small that the filter is faster.  All give the same representatives. */
 int ls_amd_set_factored_enumeration(int enable);
 int ls_amd_operator_set_schedule(ls_amd_operator *op, int lanes_f64,
                                  int flags_f64, int lanes_f32, int flags_f32);

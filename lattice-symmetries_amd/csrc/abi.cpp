@@ -977,7 +977,7 @@ extern "C" int ls_amd_operator_schedule(ls_amd_operator const *op, int *out) {
 }
 
 extern "C" int ls_amd_set_factored_enumeration(int enable) {
-  g_factored_enumeration.store(enable != 0);
+  g_factored_enumeration.store(enable);
   return 0;
 }
 

@@ -935,7 +935,7 @@ int64_t lanes_for(int64_t total, int64_t &per_lane, bool listed = false) {
 }
 } // namespace
 
-std::atomic<bool> g_factored_enumeration{true};
+std::atomic<int> g_factored_enumeration{1};
 
 namespace {
 // Scratch of the filter passes, kept between builds (grow-only) so that a
@@ -968,6 +968,30 @@ int split_low_rows(GroupData const &g) {
   int rows = g.fact_ly / 2;
   while (rows * g.fact_lx > kMaxSplitLow) --rows;
   return (g.fact_ly - rows) * g.fact_lx <= kMaxSplitHigh ? rows : 0;
+}
+
+// Whether the split enumeration is the faster one for `total` states of the
+// sector.  Its cost hardly falls with the weight: the list pass tests every
+// value of the lower rows once per top row and weight, tables over the values
+// of the upper rows are filled and scanned, and few candidates leave most
+// workgroups idle.  The filter's cost is 0.3 to 0.7 ms and then follows
+// `total`.  Measured with all reflections, filter against split, in ms:
+//   5x5  weight 5 (53 k) 0.54 / 0.61, 10 (3.3 M) 0.52 / 0.50, 12 (5.2 M) 0.47 / 0.44
+//   5x6  weight 8 (5.9 M) 0.54 / 0.59, 10 (30 M) 0.60 / 0.55, 15 (155 M) 1.1 / 0.5
+//   4x8  weight 8 (11 M) 0.58 / 0.68, 10 (65 M) 0.81 / 0.72, 16 (601 M) 3.4 / 1.0
+//   5x7  weight 8 (24 M) 0.68 / 0.78, 10 (184 M) 1.5 / 1.0
+//   6x6  weight 3 0.79 / 1.34, 8 (30 M) 0.91 / 1.20, 10 (254 M) 1.9 / 1.5, 18 (9.1 G) 39 / 4.2
+//   6x7  weight 3 0.78 / 1.58, 8 (118 M) 1.28 / 2.17
+// so the line lies at a multiple of the values that the split goes over, and
+// not below 4 M states, up to which both take launches and copies alone (on
+// lattices of at most 16 sites the split has the fewer: 0.34 against 0.38 ms).
+bool split_pays(GroupData const &g, int64_t total) {
+  if (g.number_bits <= 16) return true;
+  int const low_bits = split_low_rows(g) * g.fact_lx, high_bits = g.number_bits - low_bits;
+  int64_t tops = 0;
+  for (size_t v = 0; v < g.h_line_least.size(); ++v) tops += g.h_line_least[v] == v ? 1 : 0;
+  int64_t const listed = tops * (low_bits + 1) << low_bits, highs = int64_t{1} << high_bits;
+  return total >= std::max<int64_t>(int64_t{1} << 22, 3 * listed + 12 * highs);
 }
 
 // The split enumeration of [lower, upper]; `out` receives `kept` states.
@@ -1145,10 +1169,10 @@ bool enumerate_states(EnumerationSpec const &spec, uint64_t lower, uint64_t uppe
   bool const use_factored = q_identity >= 0;
   // The split enumeration lists the whole sector's candidates, so it serves
   // ranges of at least an eighth of the sector (it does about a tenth of the
-  // filter's work: 3.2 against 26.7 ms on 6x6).  It is the faster one at every
-  // size: 0.39 against 0.51 ms on 4x4, 0.62 against 0.91 ms on 5x6.
+  // filter's work: 3.2 against 26.7 ms on 6x6) where it pays.
   if (use_factored && g.lines() && split_low_rows(g) > 0 &&
-      static_cast<uint64_t>(p.total) >= binomial_host(n, p.hamming) / (spec.spin_inversion != 0 ? 16 : 8)) {
+      static_cast<uint64_t>(p.total) >= binomial_host(n, p.hamming) / (spec.spin_inversion != 0 ? 16 : 8) &&
+      (split_pays(g, p.total) || g_factored_enumeration.load() == 2)) {
     uint64_t kept = 0;
     timer_begin(kTimerEnumerate);
     if (!enumerate_split(g, p.hamming, lower, hi, out, kept)) return false;

@@ -60,3 +60,23 @@ def test_split_keeps_to_a_range(engine):
     low, high = int(every[every.size // 7]), int(every[-every.size // 5])
     want = every[(every >= low) & (every <= high)]
     assert np.array_equal(states(case, False, (low, high)), want)
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(map(str, c[:5])))
+def test_small_sectors_by_either_enumeration(engine, case):
+    """Sectors too small for the split to pay take the filter; forced onto the
+    split they list the same states."""
+    print(case, flush=True)
+    want = states(case, True)
+    lib = lsamd.load()
+    for mode in (1, 2):
+        lib.ls_amd_set_factored_enumeration(mode)
+        try:
+            lx, ly, weight, inversion, point, sectors = case
+            gens = torus(lx, ly, point)
+            S = lsamd.Symmetries([lsamd.Symmetry(g, s) for g, s in zip(gens, sectors or [0] * len(gens))])
+            basis = lsamd.DeviceBasis(lx * ly, weight, inversion, S)
+            basis.build()
+        finally:
+            lib.ls_amd_set_factored_enumeration(1)
+        assert np.array_equal(basis.states, want)
