@@ -132,43 +132,54 @@ __global__ __launch_bounds__(256) void species_compact_kernel(uint32_t const *__
   if (s < states && flags[s] != 0) out[places[s]] = static_cast<uint32_t>(s);
 }
 
+// Acceptance bits of the products (one word a wave) and how many a workgroup
+// accepts: a fifth of a byte of scratch per product.
 template <typename W, int D>
 __global__ __launch_bounds__(256) void species_count_kernel(GroupView g, uint32_t const *__restrict__ downs,
                                                             uint32_t const *__restrict__ ups, int64_t nup,
-                                                            int64_t total, uint32_t *__restrict__ flags) {
+                                                            int64_t total, uint64_t *__restrict__ bits,
+                                                            uint32_t *__restrict__ counts) {
   extern __shared__ uint64_t search_lds[];
   SpeciesSearch<W, D> search;
   search.stage(g, search_lds);
   __syncthreads();
   int64_t const c = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (c >= total) return;
-  uint32_t const down = downs[c / nup], up = ups[c % nup];
-  int const words = ((1 << (g.nbits / 2)) + 31) / 32;
-  uint64_t const entry = g.species_entry[down];
-  int const count = static_cast<int>(entry >> 16 & 0xffffu);
-  uint16_t const *list = g.species_list + (entry >> 32);
-  int sum = 0;
-  bool ok = true;
-  for (int i = 0; i < count && ok; ++i) {
-    int const e = list[i];
-    W const y = search.up_image(g, e, static_cast<W>(up));
-    ok = y >= static_cast<W>(up);
-    if (y == static_cast<W>(up)) {
-      bool const minus = search.odd(g, e, up, words) != search.odd(g, e, down, words);
-      sum += (g.eig_re[e] < 0.0) != minus ? -1 : 1;
+  bool ok = c < total;
+  if (ok) {
+    uint32_t const down = downs[c / nup], up = ups[c % nup];
+    int const words = ((1 << (g.nbits / 2)) + 31) / 32;
+    uint64_t const entry = g.species_entry[down];
+    int const count = static_cast<int>(entry >> 16 & 0xffffu);
+    uint16_t const *list = g.species_list + (entry >> 32);
+    int sum = 0;
+    for (int i = 0; i < count && ok; ++i) {
+      int const e = list[i];
+      W const y = search.up_image(g, e, static_cast<W>(up));
+      ok = y >= static_cast<W>(up);
+      if (y == static_cast<W>(up)) {
+        bool const minus = search.odd(g, e, up, words) != search.odd(g, e, down, words);
+        sum += (g.eig_re[e] < 0.0) != minus ? -1 : 1;
+      }
     }
+    ok = ok && static_cast<double>(sum) > g.norm_eps;
   }
-  flags[c] = ok && static_cast<double>(sum) > g.norm_eps ? 1u : 0u;
+  uint64_t const mask = __ballot(ok);
+  if ((threadIdx.x & 63) == 0) bits[c >> 6] = mask;
+  int const accepted = __syncthreads_count(ok);
+  if (threadIdx.x == 0) counts[blockIdx.x] = static_cast<uint32_t>(accepted);
 }
 
 __global__ __launch_bounds__(256) void species_write_kernel(uint32_t const *__restrict__ downs,
                                                             uint32_t const *__restrict__ ups, int64_t nup,
-                                                            int64_t total, int sites,
-                                                            uint32_t const *__restrict__ flags,
-                                                            uint64_t const *__restrict__ places,
+                                                            int sites, uint64_t const *__restrict__ bits,
+                                                            uint64_t const *__restrict__ offsets,
                                                             uint64_t *__restrict__ out) {
   int64_t const c = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (c < total && flags[c] != 0) out[places[c]] = static_cast<uint64_t>(downs[c / nup]) << sites | ups[c % nup];
+  uint64_t const word = bits[c >> 6];
+  if ((word >> (c & 63) & 1u) == 0) return;
+  uint64_t o = offsets[blockIdx.x] + static_cast<uint64_t>(__popcll(word & ((uint64_t{1} << (c & 63)) - 1)));
+  for (int64_t w = static_cast<int64_t>(blockIdx.x) * 4; w < c >> 6; ++w) o += static_cast<uint64_t>(__popcll(bits[w]));
+  out[o] = static_cast<uint64_t>(downs[c / nup]) << sites | ups[c % nup];
 }
 
 bool enumerate_species(GroupData const &g, uint64_t min_up, uint64_t max_up, uint64_t min_down, uint64_t max_down,
@@ -198,23 +209,26 @@ bool enumerate_species(GroupData const &g, uint64_t min_up, uint64_t max_up, uin
     size[down] = static_cast<int64_t>(count);
   }
   int64_t const total = size[0] * size[1];
-  DeviceArray<uint32_t> accepted;
-  DeviceArray<uint64_t> offsets;
-  if (!accepted.allocate(static_cast<size_t>(total)) || !offsets.allocate(static_cast<size_t>(total))) return false;
+  int const groups = grid_for(total, 256);
+  DeviceArray<uint32_t> counts;
+  DeviceArray<uint64_t> bits, offsets;
+  if (!bits.allocate(4 * static_cast<size_t>(groups)) || !counts.allocate(static_cast<size_t>(groups)) ||
+      !offsets.allocate(static_cast<size_t>(groups)))
+    return false;
   bool const ok = dispatch_group(g, [&]<typename W, int D, int SI>() -> bool {
     if constexpr (SI == kFermionic) {
-      species_count_kernel<W, D><<<grid_for(total, 256), 256, species_lds_bytes(g), stream()>>>(
-          v, list[1].ptr, list[0].ptr, size[0], total, accepted.ptr);
+      species_count_kernel<W, D><<<groups, 256, species_lds_bytes(g), stream()>>>(
+          v, list[1].ptr, list[0].ptr, size[0], total, bits.ptr, counts.ptr);
       LSAMD_HIP(hipGetLastError());
       return true;
     }
     return fail("species tables need a fermionic group");
   });
-  if (!ok || !exclusive_scan(accepted.ptr, total, offsets.ptr, kept) || !out.allocate(static_cast<size_t>(kept)))
+  if (!ok || !exclusive_scan(counts.ptr, groups, offsets.ptr, kept) || !out.allocate(static_cast<size_t>(kept)))
     return false;
   if (kept > 0) {
-    species_write_kernel<<<grid_for(total, 256), 256, 0, stream()>>>(list[1].ptr, list[0].ptr, size[0], total, sites,
-                                                                     accepted.ptr, offsets.ptr, out.ptr);
+    species_write_kernel<<<groups, 256, 0, stream()>>>(list[1].ptr, list[0].ptr, size[0], sites, bits.ptr, offsets.ptr,
+                                                       out.ptr);
     LSAMD_HIP(hipGetLastError());
   }
   LSAMD_HIP(hipStreamSynchronize(stream()));

@@ -92,3 +92,20 @@ def test_species_basis_and_matrix(engine, name, gens, sectors):
             op.build_csr(128)
         for a, b in zip(fast.csr_arrays(), slow.csr_arrays()):
             assert np.array_equal(a, b)
+
+
+def test_species_basis_takes_little_scratch(engine):
+    """A trivial group on 16 sites lists every product: 23 M states, whose
+    scratch has to stay far below their own 8 bytes each."""
+    n = 16
+    S = lsamd.Symmetries([lsamd.Symmetry(np.arange(2 * n, dtype=np.int32), 0)])
+    basis = lsamd.DeviceBasis.fermions(n, 4, 8, S)
+    lsamd.device_trim()
+    basis.build()
+    assert lsamd.device_trim() <= basis.number_states
+    states = basis.states
+    assert basis.number_states == 1820 * 12870
+    assert np.all(np.diff(states.view(np.int64)) > 0)
+    low = np.uint64((1 << n) - 1)
+    for species, weight in ((states & low, 4), (states >> np.uint64(n), 8)):
+        assert np.all(np.unpackbits(species.view(np.uint8).reshape(-1, 8), axis=1).sum(axis=1) == weight)
