@@ -542,8 +542,11 @@ constexpr int kMaxProbes = 128;
 struct ValueHash {
   unsigned long long *slots; // [kValueSlots]
   int *distinct;             // values inserted
-  int *overflow;             // more than kWideTableSize of them, or a target row too long for a tag
+  int *overflow;             // kManyValues, kLongRow
 };
+// Why a kFillTable pass stops: more than kWideTableSize values, or a target row
+// too long for a tag's place bits.
+constexpr int kManyValues = 1, kLongRow = 2;
 
 __device__ __forceinline__ uint32_t slot_hash(uint64_t k) {
   k ^= k >> 33;
@@ -562,14 +565,14 @@ __device__ __forceinline__ uint32_t value_slot(ValueHash const &h, double v) {
     if (cur == kEmptySlot) {
       cur = atomicCAS(&h.slots[slot], static_cast<unsigned long long>(kEmptySlot), key);
       if (cur == kEmptySlot) {
-        if (atomicAdd(h.distinct, 1) >= kWideTableSize) atomicExch(h.overflow, 1);
+        if (atomicAdd(h.distinct, 1) >= kWideTableSize) atomicOr(h.overflow, kManyValues);
         return slot;
       }
     }
     if (cur == key) return slot;
     slot = (slot + 1) & (kValueSlots - 1);
   }
-  atomicExch(h.overflow, 1);
+  atomicOr(h.overflow, kLongRow); // a crowded stretch of a table with room: the values may still be few
   return 0;
 }
 
@@ -626,7 +629,7 @@ __global__ __launch_bounds__(kPairThreads) void csr_fill_kernel(GroupView g, OpV
       cols[o] = col;
       if (col != kDropped) {
         uint32_t const place = atomicAdd(&targets[col], 1u);
-        if (place >> kTagPlaceBits != 0) atomicExch(hash.overflow, 1);
+        if (place >> kTagPlaceBits != 0) atomicOr(hash.overflow, kLongRow);
         tags[o] = (value_slot(hash, c_re) << kTagPlaceBits | (place & ((1u << kTagPlaceBits) - 1))) << kTagRowBits |
                   static_cast<uint32_t>(r);
       }
@@ -1273,11 +1276,11 @@ __global__ __launch_bounds__(256) void split_wide_keys_kernel(int64_t nnz, uint6
 // writes, and a sort of 6 ms replace a counting pass (28 ms), a scatter of
 // 8-byte keys through atomic cursors (42 ms), their LDS sort (24 ms), a gather
 // of the values in target order (23 ms), the distinct-value pass and the
-// packing (11 ms), and the temporaries shrink from 28 to 14 GB.  `done` stays false when the matrix has too many values, a
-// target row of more than 4096 entries, or no entries: then the general
-// build runs.
-bool build_table_csr(OperatorCore &op, int64_t up, int64_t const *row_ptr, bool &done) {
-  done = false;
+// packing (11 ms), and the temporaries shrink from 28 to 14 GB.  `done` stays
+// false when the matrix has too many values (`many`), a target row of more than
+// 4096 entries, or no entries: then the general build runs.
+bool build_table_csr(OperatorCore &op, int64_t up, int64_t const *row_ptr, bool &done, bool &many) {
+  done = many = false;
   int64_t const n = op.number_states;
   Csr &c = op.csr;
   DeviceArray<uint32_t> cols, tags, targets;
@@ -1305,6 +1308,7 @@ bool build_table_csr(OperatorCore &op, int64_t up, int64_t const *row_ptr, bool 
   LSAMD_HIP(hipStreamSynchronize(stream()));
   if (h_flags[1] != 0) { // the general build goes over every pair again and reports what it finds
     LSAMD_HIP(hipMemsetAsync(op.d_err.ptr, 0, sizeof(int), stream()));
+    many = (h_flags[1] & kManyValues) != 0;
     return true;
   }
   if (!check_error(op)) return false;
@@ -1447,8 +1451,8 @@ bool operator_build_csr(OperatorCore &op, int precision) {
   }
   DeviceArray<uint32_t> cols;
   DeviceArray<double> vals;
-  bool table = false;
-  if (!cplx && op.allow_packing && up > 0 && !build_table_csr(op, up, row_ptr.ptr, table)) return false;
+  bool table = false, many = false;
+  if (!cplx && op.allow_packing && up > 0 && !build_table_csr(op, up, row_ptr.ptr, table, many)) return false;
   if (table) {
     timer_end(kTimerCsrBuild);
     return finish_real_csr(op, precision, vals);
@@ -1510,7 +1514,7 @@ bool operator_build_csr(OperatorCore &op, int precision) {
     LSAMD_HIP(hipStreamSynchronize(stream()));
     return true;
   }
-  if (op.allow_packing && !try_pack_values(c, vals.ptr)) return false;
+  if (op.allow_packing && !many && !try_pack_values(c, vals.ptr)) return false;
   return finish_real_csr(op, precision, vals);
 }
 

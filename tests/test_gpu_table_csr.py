@@ -153,3 +153,13 @@ def test_a_full_value_hash_still_reports_states_outside_the_basis(engine):
             op.build_csr(64)
     good = lsamd.DeviceOperator(b, models.heisenberg_chain(16))
     assert good.build_csr(64) > 0
+
+
+def test_a_long_row_of_few_values_is_still_packed(engine):
+    """The table pass gives up on a row too long for its tags; the general
+    build then packs the few values."""
+    b, expr = CASES["flips4500"]()
+    op = lsamd.DeviceOperator(b, expr)
+    op.build_csr(64)
+    info = op.csr_info
+    assert info["packed"] and info["table_size"] == len(set(expr.terms.values()))
