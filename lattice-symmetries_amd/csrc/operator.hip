@@ -732,13 +732,13 @@ __global__ __launch_bounds__(256) void push_scatter_kernel(int64_t n, int64_t co
   }
 }
 
-template <typename Key> __device__ void heap_sort(Key *a, int64_t n) {
-  auto sift = [a](int64_t root, int64_t end) {
+template <typename Key, typename Less> __device__ void heap_sort(Key *a, int64_t n, Less const &less) {
+  auto sift = [a, &less](int64_t root, int64_t end) {
     while (true) {
       int64_t child = 2 * root + 1;
       if (child >= end) return;
-      if (child + 1 < end && a[child] < a[child + 1]) ++child;
-      if (a[root] >= a[child]) return;
+      if (child + 1 < end && less(a[child], a[child + 1])) ++child;
+      if (!less(a[root], a[child])) return;
       Key const t = a[root];
       a[root] = a[child];
       a[child] = t;
@@ -780,12 +780,24 @@ __device__ __forceinline__ double key_value(uint64_t key, int64_t const *src_ptr
   return vals[src_ptr[key >> kKeyLocalBits] + static_cast<int64_t>(key & ((uint64_t{1} << kKeyLocalBits) - 1))];
 }
 
+// One lane orders a run: by insertion while that is short (a run is as many
+// terms as take one state to the same other one; a 1-state basis with 2000 of
+// them took 160 ms so, 64-entry runs about as long either way).
+constexpr int kInsertionRun = 64;
+
 __device__ __forceinline__ void order_ties(uint64_t *a, int64_t len, int64_t const *src_ptr, double const *vals) {
   int const shift = src_ptr == nullptr ? 32 : kKeyLocalBits;
   for (int64_t q = threadIdx.x; q + 1 < len; q += 64) {
     uint64_t const i = a[q] >> shift;
     if ((q > 0 && (a[q - 1] >> shift) == i) || (a[q + 1] >> shift) != i) continue; // not the start of a run
-    for (int64_t t = q + 1; t < len && (a[t] >> shift) == i; ++t) {
+    int64_t end = q + 2;
+    while (end < len && (a[end] >> shift) == i) ++end;
+    if (end - q > kInsertionRun) {
+      heap_sort(a + q, end - q,
+                [&](uint64_t x, uint64_t y) { return key_value(x, src_ptr, vals) < key_value(y, src_ptr, vals); });
+      continue;
+    }
+    for (int64_t t = q + 1; t < end; ++t) {
       uint64_t const key = a[t];
       double const v = key_value(key, src_ptr, vals);
       int64_t u = t;
@@ -816,7 +828,7 @@ __global__ __launch_bounds__(64) void sort_rows_kernel(int64_t n, int64_t const 
     int64_t const len = rp[row + 1] - b;
     if (len <= min_len) continue;
     if (len > cap) {
-      if (threadIdx.x == 0) heap_sort(keys + b, len);
+      if (threadIdx.x == 0) heap_sort(keys + b, len, [](Key x, Key y) { return x < y; });
       __syncthreads();
       if constexpr (sizeof(Key) == 8) {
         if (vals != nullptr) order_ties(keys + b, len, src_ptr, vals);

@@ -163,3 +163,31 @@ def test_a_long_row_of_few_values_is_still_packed(engine):
     op.build_csr(64)
     info = op.csr_info
     assert info["packed"] and info["table_size"] == len(set(expr.terms.values()))
+
+
+def same_target_hops(count, seed):
+    """`count` terms, all of which take the one-particle orbit of the 4x4
+    lattice to itself: hops from site 0 with other sites asked to be empty."""
+    values = np.random.default_rng(seed).permutation(count) / 1024.0 + 1.0
+    out = {}
+    for q in range(count):
+        j, sub = 1 + q % 15, q // 15
+        rest = [s for s in range(1, 16) if s != j]
+        m = 1 | 1 << j | sum((sub >> p & 1) << s for p, s in enumerate(rest))
+        out[(m, 1 << j, 1, 1 | 1 << j, 0)] = float(values[q])
+    return Expr(out)
+
+
+@pytest.mark.parametrize("count", [2, 63, 64, 65, 66, 300, 1024, 1025, 3000])
+def test_many_entries_of_one_column_in_ascending_value(engine, count):
+    """Both builds list a column's entries in ascending value, whatever sort a
+    run of them takes (one row of `count` entries)."""
+    b = torus_basis(4, 1)
+    expr = same_target_hops(count, count)
+    for packing in (True, False):
+        op = lsamd.DeviceOperator(b, expr)
+        op.set_csr_packing(packing)
+        assert op.build_csr(64) == count
+        rows, cols, vals, _ = op.csr_arrays()
+        assert list(rows) == [0, count] and not cols.any()
+        assert np.array_equal(vals, np.sort(np.array(list(expr.terms.values())).real))
