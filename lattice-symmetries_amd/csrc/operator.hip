@@ -337,7 +337,8 @@ __device__ __forceinline__ void off_diag_entry(GroupView const &g, OpView const 
     // BatchedOperator.chpl:232-247
     StateInfo const s = search.info(g, beta);
     double const t_re = (re * s.norm) / n_alpha;
-    double const t_im = im != 0.0 ? (im * s.norm) / n_alpha : im;
+    // a real term skips the division unless it would give NaN (a listed state of norm 0)
+    double const t_im = im != 0.0 || !(n_alpha > 0.0) ? (im * s.norm) / n_alpha : im;
     re = s.c_re * t_re - s.c_im * t_im;
     im = s.c_re * t_im + s.c_im * t_re;
     beta = s.rep;

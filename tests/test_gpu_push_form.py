@@ -188,3 +188,36 @@ def test_non_hermitian_sector_batch(engine):
         off += dim
     with pytest.raises(lsamd.EngineError, match="not Hermitian"):
         batch.eigensolve(nev=1, block_size=1, max_blocks=4, keep_blocks=2)
+
+
+def listed_minima():
+    """Every orbit minimum of the 10-site chain at half filling, among them the
+    reflection-symmetric ones, whose norm in the odd sector is 0."""
+    n = 10
+    gens = [models.chain_translation(n), models.chain_parity(n)]
+    S = lsamd.Symmetries([lsamd.Symmetry(g, s) for g, s in zip(gens, [0, 1])])
+    og = O.Group(n, S.elements(), S.characters.real, S.characters.imag, 0)
+    xs = np.array([x for x in range(1 << n) if bin(x).count("1") == n // 2], dtype=np.uint64)
+    reps, _, norms = og.state_info(xs)
+    minima = xs[reps == xs]
+    assert 0 < np.count_nonzero(norms[reps == xs] == 0.0) < minima.size
+    return n, S, og, minima
+
+
+def test_listed_states_of_norm_zero(engine):
+    """c n_beta / n_alpha of a listed state of norm 0 is NaN in the reference,
+    also for a real term: complex multiplication by the character meets 0 / 0."""
+    n, S, og, minima = listed_minima()
+    basis = lsamd.DeviceBasis(n, n // 2, None, S)
+    basis.set_states(minima)
+    expr = sigma_plus(4) * sigma_minus(2)  # one term: no two infinities meet in a sum
+    diag, off = expr.split()
+    x = np.random.default_rng(3).standard_normal(minima.size)
+    want = O.matvec_push(og, n, 0, minima, O.Terms(diag), O.Terms(off), x)
+    assert np.isnan(want).any() and not np.isinf(want).any()
+    for factored in (True, False):
+        op = lsamd.DeviceOperator(basis, expr)
+        op.set_factored(factored)
+        got = op.matvec(x, "otf")
+        say(factored, np.isnan(want).sum(), np.isnan(got).sum(), np.isinf(got).sum())
+        assert np.allclose(got, want, rtol=RTOL64, atol=RTOL64 * np.nanmax(np.abs(want)), equal_nan=True)
