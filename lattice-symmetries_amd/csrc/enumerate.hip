@@ -976,12 +976,12 @@ int split_low_rows(GroupData const &g) {
 // of the upper rows are filled and scanned, and few candidates leave most
 // workgroups idle.  The filter's cost is 0.3 to 0.7 ms and then follows
 // `total`.  Measured with all reflections, filter against split, in ms:
-//   5x5  weight 5 (53 k) 0.54 / 0.61, 10 (3.3 M) 0.52 / 0.50, 12 (5.2 M) 0.47 / 0.44
-//   5x6  weight 8 (5.9 M) 0.54 / 0.59, 10 (30 M) 0.60 / 0.55, 15 (155 M) 1.1 / 0.5
+//   5x5  weight 5 (53 k) 0.53 / 0.61, 10 (3.3 M) 0.50 / 0.50, 12 (5.2 M) 0.47 / 0.44
+//   5x6  weight 8 (5.9 M) 0.53 / 0.59, 10 (30 M) 0.60 / 0.55, 15 (155 M) 1.1 / 0.5
 //   4x8  weight 8 (11 M) 0.58 / 0.68, 10 (65 M) 0.81 / 0.72, 16 (601 M) 3.4 / 1.0
-//   5x7  weight 8 (24 M) 0.68 / 0.78, 10 (184 M) 1.5 / 1.0
-//   6x6  weight 3 0.79 / 1.34, 8 (30 M) 0.91 / 1.20, 10 (254 M) 1.9 / 1.5, 18 (9.1 G) 39 / 4.2
-//   6x7  weight 3 0.78 / 1.58, 8 (118 M) 1.28 / 2.17
+//   5x7  weight 8 (24 M) 0.67 / 0.78, 10 (184 M) 1.5 / 1.0
+//   6x6  weight 3 0.73 / 1.34, 8 (30 M) 0.82 / 1.20, 10 (254 M) 1.9 / 1.5, 18 (9.1 G) 39 / 4.2
+//   6x7  weight 3 0.71 / 1.58, 8 (118 M) 1.22 / 2.17
 // so the line lies at a multiple of the values that the split goes over, and
 // not below 4 M states, up to which both take launches and copies alone (on
 // lattices of at most 16 sites the split has the fewer: 0.34 against 0.38 ms).

@@ -388,12 +388,18 @@ bool group_plan_lines(GroupData &g, std::vector<Perm> const &perms) {
   uint8_t *const rot = raw + g.line_off_rot;
   std::memcpy(raw + g.line_off_q, line_q.data(), line_q.size() * sizeof(int32_t));
   uint32_t const rm = static_cast<uint32_t>(nv) - 1;
+  std::vector<uint8_t> first(2 * static_cast<size_t>(nv), 0xff), reach(first.size(), 0); // least rotation, and which give it
   for (int mirror = 0; mirror < 2; ++mirror)
     for (int v = 0; v < nv; ++v) {
       uint32_t w = 0;
       for (int c = 0; c < lx; ++c) w |= ((static_cast<uint32_t>(v) >> (mirror ? (lx - c) % lx : c)) & 1u) << c;
-      for (int a = 0; a < lx; ++a)
-        rot[(mirror * lx + a) * nv + v] = static_cast<uint8_t>(((w >> a) | (w << (lx - a))) & rm);
+      uint8_t &least = first[mirror * nv + v], &at = reach[mirror * nv + v];
+      for (int a = 0; a < lx; ++a) {
+        auto const r = static_cast<uint8_t>(((w >> a) | (w << (lx - a))) & rm);
+        rot[(mirror * lx + a) * nv + v] = r;
+        at = static_cast<uint8_t>((r < least ? 0 : at) | (r <= least ? 1 << a : 0));
+        least = std::min(least, r);
+      }
     }
   for (int k = 1; k < nc; ++k) {
     size_t const e = static_cast<size_t>(g.h_fact_q[bases[k]]) * g.depth;
@@ -412,8 +418,11 @@ bool group_plan_lines(GroupData &g, std::vector<Perm> const &perms) {
       for (int s = 0; s < flips; ++s) {
         uint32_t const x = s ? rm : 0, top = ((v & 2) ? lower : upper) ^ x, next = ((v & 2) ? upper : lower) ^ x;
         uint8_t const *r = rot + static_cast<size_t>(v & 1) * lx * nv;
-        for (int a = 0; a < lx; ++a) {
-          uint32_t const k = (static_cast<uint32_t>(r[a * nv + top]) << lx) | r[a * nv + next];
+        uint32_t const lead = static_cast<uint32_t>(first[(v & 1) * nv + top]) << lx;
+        if (lead > least) continue;
+        for (uint32_t at = reach[(v & 1) * nv + top]; at != 0; at &= at - 1) {
+          int const a = __builtin_ctz(at);
+          uint32_t const k = lead | r[a * nv + next];
           if (k < least) {
             least = k;
             mask = 0;
