@@ -104,10 +104,12 @@ __global__ __launch_bounds__(kThreads) void sector_spmv_kernel(int64_t n, int64_
   }
   // As in csr_block_rows, several lanes share an entry: each takes kPart
   // columns, 16 bytes of the real and of the imaginary parts where K allows.
-  // 52 sectors of the 26-site chain, 8 columns: FP32 2.84 -> 2.43 ms, FP64 6.94
-  // -> 3.88 ms; two or four entries in flight per lane gain nothing more (2.52,
-  // 2.66 ms: rows of 27 entries leave remainders).  Bound by the L2 misses of
-  // the x rows and the 12 (20) bytes of column and value per entry.
+  // 52 sectors of the 26-site chain, 8 columns: FP32 2.78 -> 2.36 ms (J1-J2),
+  // FP64 3.80 -> 2.51 ms (J1 alone).  A loop over kShare whole entries before the
+  // remainder is slower (2.45 ms: rows of 27 entries leave remainders), one
+  // chain of sums 1 to 5 % faster but less exact.  Not limited by arithmetic:
+  // it gathers x rows that miss L2 and streams 12 (20) bytes of column and value
+  // per entry.
   constexpr int kWant = static_cast<int>(sizeof(T)) * K / 16;
   constexpr int kShare = kWant < 1 ? 1 : (kWant < LPR ? kWant : LPR);
   constexpr int kPart = K / kShare;
@@ -118,29 +120,47 @@ __global__ __launch_bounds__(kThreads) void sector_spmv_kernel(int64_t n, int64_
   T const *__restrict__ xp = x + sub % kShare * kPart;
   for (; t < t_end; t += t_step) {
     int64_t const row = t * kRows + r_in;
-    T re[kPart], im[kPart];
+    T res[kShare][kPart], ims[kShare][kPart]; // one chain of sums per lane that shares an entry, as in csr_block_rows
 #pragma unroll
-    for (int q = 0; q < kPart; ++q) re[q] = im[q] = T(0);
+    for (int u = 0; u < kShare; ++u)
+#pragma unroll
+      for (int q = 0; q < kPart; ++q) res[u][q] = ims[u][q] = T(0);
     if (row < n) {
       int64_t const b = rp[row], e = rp[row + 1];
-      for (int64_t k = b + sub / kShare; k < e; k += kStep) {
-        T2 const v = v2[k];
-        T const *__restrict__ xr = xp + static_cast<size_t>(cols[k]) * (2 * K);
-        T xre[kPart], xim[kPart];
+      for (int64_t k0 = b + sub / kShare; k0 < e; k0 += kShare * kStep) {
 #pragma unroll
-        for (int q = 0; q < kPart; ++q) {
-          xre[q] = xr[q];
-          xim[q] = xr[K + q];
-        }
+        for (int u = 0; u < kShare; ++u) {
+          int64_t const k = k0 + u * kStep;
+          if (u > 0 && k >= e) break;
+          T2 const v = v2[k];
+          T const *__restrict__ xr = xp + static_cast<size_t>(cols[k]) * (2 * K);
+          T xre[kPart], xim[kPart];
 #pragma unroll
-        for (int q = 0; q < kPart; ++q) {
-          re[q] = fma(v.x, xre[q], re[q]);
-          re[q] = fma(-v.y, xim[q], re[q]);
-          im[q] = fma(v.y, xre[q], im[q]);
-          im[q] = fma(v.x, xim[q], im[q]);
+          for (int q = 0; q < kPart; ++q) {
+            xre[q] = xr[q];
+            xim[q] = xr[K + q];
+          }
+#pragma unroll
+          for (int q = 0; q < kPart; ++q) {
+            res[u][q] = fma(v.x, xre[q], res[u][q]);
+            res[u][q] = fma(-v.y, xim[q], res[u][q]);
+            ims[u][q] = fma(v.y, xre[q], ims[u][q]);
+            ims[u][q] = fma(v.x, xim[q], ims[u][q]);
+          }
         }
       }
     }
+#pragma unroll
+    for (int c = kShare / 2; c > 0; c >>= 1)
+#pragma unroll
+      for (int u = 0; u < c; ++u)
+#pragma unroll
+        for (int q = 0; q < kPart; ++q) {
+          res[u][q] += res[u + c][q];
+          ims[u][q] += ims[u + c][q];
+        }
+    T(&re)[kPart] = res[0];
+    T(&im)[kPart] = ims[0];
 #pragma unroll
     for (int q = 0; q < kPart; ++q) {
 #pragma unroll

@@ -186,6 +186,11 @@ __device__ __forceinline__ void csr_block_rows(int64_t n, int64_t const *__restr
   constexpr int kPart = K / kShare;                                   // values of a lane
   constexpr int kStep = LPR / kShare;                                 // entries of a row at a time
   constexpr int kAhead = 4;
+  // Shared lanes meet kShare times as many entries of a row; they sum them in
+  // as many chains, no longer than those of lanes with an entry of their own.
+  // With one chain the FP32 block of 8 rounded worse (28-site chain, relative
+  // error 7.05e-8 against 6.16e-8) and took the same 9.21 ms on 6x6.
+  constexpr int kChains = kShare < kAhead ? kShare : kAhead;
   int64_t const tiles = (n + kRows - 1) / kRows;
   int64_t t, t_end, t_step;
   tile_range<DIE>(tiles, t, t_end, t_step);
@@ -193,9 +198,11 @@ __device__ __forceinline__ void csr_block_rows(int64_t n, int64_t const *__restr
   T const *__restrict__ xp = x + sub % kShare * kPart;
   for (; t < t_end; t += t_step) {
     int64_t const row = t * kRows + static_cast<int>(threadIdx.x) / LPR;
-    T acc[kPart];
+    T sum[kChains][kPart];
 #pragma unroll
-    for (int q = 0; q < kPart; ++q) acc[q] = T(0);
+    for (int u = 0; u < kChains; ++u)
+#pragma unroll
+      for (int q = 0; q < kPart; ++q) sum[u][q] = T(0);
     if (row < n) {
       int64_t const b = rp[row], e = rp[row + 1];
       int64_t k = b + first;
@@ -212,17 +219,28 @@ __device__ __forceinline__ void csr_block_rows(int64_t n, int64_t const *__restr
 #pragma unroll
         for (int u = 0; u < kAhead; ++u)
 #pragma unroll
-          for (int q = 0; q < kPart; ++q) acc[q] = fma(v[u], a[u][q], acc[q]);
+          for (int q = 0; q < kPart; ++q) sum[u % kChains][q] = fma(v[u], a[u][q], sum[u % kChains][q]);
       }
-      for (; k < e; k += kStep) {
-        uint32_t col;
-        T v;
-        ent(k, col, v);
-        T const *xr = xp + static_cast<size_t>(col) * K;
+      for (; k < e; k += kChains * kStep) {
 #pragma unroll
-        for (int q = 0; q < kPart; ++q) acc[q] = fma(v, xr[q], acc[q]);
+        for (int u = 0; u < kChains; ++u) {
+          if (u > 0 && k + u * kStep >= e) break;
+          uint32_t col;
+          T v;
+          ent(k + u * kStep, col, v);
+          T const *xr = xp + static_cast<size_t>(col) * K;
+#pragma unroll
+          for (int q = 0; q < kPart; ++q) sum[u][q] = fma(v, xr[q], sum[u][q]);
+        }
       }
     }
+#pragma unroll
+    for (int c = kChains / 2; c > 0; c >>= 1)
+#pragma unroll
+      for (int u = 0; u < c; ++u)
+#pragma unroll
+        for (int q = 0; q < kPart; ++q) sum[u][q] += sum[u + c][q];
+    T(&acc)[kPart] = sum[0];
 #pragma unroll
     for (int q = 0; q < kPart; ++q)
 #pragma unroll
