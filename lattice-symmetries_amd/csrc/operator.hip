@@ -556,19 +556,40 @@ __device__ __forceinline__ uint32_t slot_hash(uint64_t k) {
   return static_cast<uint32_t>(k);
 }
 
+__device__ __forceinline__ uint64_t lane_value(uint64_t v, int lane) {
+  return static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v >> 32), lane))) << 32 |
+         static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), lane));
+}
+
 // Slot of a value, inserted when new.  A plain load that finds the value or a
-// stale empty slot is enough: the exchange decides.
+// stale empty slot is enough: the exchange decides.  When a pass starts every
+// lane meets the same few new values at once, so the lanes of a wave that hold
+// one value make one exchange (the first kGroups values; lanes with others one
+// each): without, 16 to 20 sites without a group (one value) built in 0.64 to
+// 1.19 ms instead of 0.41 to 0.52.
+constexpr int kGroups = 4;
+
 __device__ __forceinline__ uint32_t value_slot(ValueHash const &h, double v) {
   unsigned long long const key = static_cast<unsigned long long>(__double_as_longlong(v));
   uint32_t slot = slot_hash(key) & (kValueSlots - 1);
+  int const lane = static_cast<int>(threadIdx.x) & 63;
   for (int probe = 0; probe < kMaxProbes; ++probe) {
     unsigned long long cur = h.slots[slot];
     if (cur == kEmptySlot) {
-      cur = atomicCAS(&h.slots[slot], static_cast<unsigned long long>(kEmptySlot), key);
-      if (cur == kEmptySlot) {
-        if (atomicAdd(h.distinct, 1) >= kWideTableSize) atomicOr(h.overflow, kManyValues);
-        return slot;
+      int leader = lane;
+      uint64_t pending = __ballot(true);
+      for (int g = 0; g < kGroups && pending != 0; ++g) {
+        int const l = __ffsll(static_cast<unsigned long long>(pending)) - 1;
+        bool const same = key == lane_value(key, l) && slot == static_cast<uint32_t>(lane_value(slot, l));
+        leader = same ? l : leader;
+        pending &= ~__ballot(same);
       }
+      if (leader == lane) {
+        cur = atomicCAS(&h.slots[slot], static_cast<unsigned long long>(kEmptySlot), key);
+        if (cur == kEmptySlot && atomicAdd(h.distinct, 1) >= kWideTableSize) atomicOr(h.overflow, kManyValues);
+      }
+      cur = __shfl(cur, leader, 64);
+      if (cur == kEmptySlot) return slot;
     }
     if (cur == key) return slot;
     slot = (slot + 1) & (kValueSlots - 1);

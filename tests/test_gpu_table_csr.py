@@ -191,3 +191,21 @@ def test_many_entries_of_one_column_in_ascending_value(engine, count):
         rows, cols, vals, _ = op.csr_arrays()
         assert list(rows) == [0, count] and not cols.any()
         assert np.array_equal(vals, np.sort(np.array(list(expr.terms.values())).real))
+
+
+@pytest.mark.parametrize("count", [1, 2, 4, 5, 63, 64, 65, 300])
+def test_values_met_by_all_waves_at_once_are_counted_once(engine, count):
+    """`count` values over 1024 terms: up to kGroups (4) values of a wave are
+    inserted by one lane each, further ones by every lane that holds them."""
+    b = basis(16)
+    values = [1.0 + (k % count) / 512.0 for k in range(1024)]
+    expr = Expr(dict(zip(projected_flips(1024).terms, values)))
+    plain = lsamd.DeviceOperator(b, expr)
+    plain.set_csr_packing(False)
+    nnz = plain.build_csr(64)
+    for _ in range(3):
+        op = lsamd.DeviceOperator(b, expr)
+        assert op.build_csr(64) == nnz
+        assert op.csr_info["table_size"] == count
+        for got, want in zip(op.csr_arrays(), plain.csr_arrays()):
+            assert np.array_equal(got, want)
