@@ -92,11 +92,15 @@ bool launch_state_index(IndexView const &idx, int64_t count, uint64_t const *d_x
   return true;
 }
 
-// offsets[b] = first position whose state has prefix >= b (b = 0 .. 2^P).  A
-// workgroup owns kPrefixBlock entries: one thread each searches the whole list
-// for its first and its end, and the entries between search only what lies
-// between those two (nothing, for the many prefixes no representative has).
-// 6x6 (2^26 entries): 0.75 ms with every entry searching the list.
+// offsets[b] = first position whose state has prefix >= b (b = 0 .. 2^P).
+// BOUNDED: a workgroup owns kPrefixBlock entries; one thread each searches the
+// whole list for its first and its end, and the entries between search only
+// what lies between those two (nothing, for the many prefixes no representative
+// has).  6x6 (2^26 entries): 0.75 -> 0.17 ms, 24 sites without a group (2^24)
+// 0.10 ms less.  Up to 2^20 entries the two searches in a row take longer than
+// a search of the list by every entry (bases of 4096 to 262 144 states 55-60
+// against 48-53 us, 2^20 equal).
+constexpr int64_t kDirectPrefixTable = int64_t{1} << 20;
 constexpr int kPrefixBlock = 1024;
 
 __device__ __forceinline__ int64_t first_with_prefix(uint64_t const *__restrict__ reps, int64_t lo, int64_t n, int shift,
@@ -110,10 +114,17 @@ __device__ __forceinline__ int64_t first_with_prefix(uint64_t const *__restrict_
   return lo;
 }
 
+template <bool BOUNDED>
 __global__ __launch_bounds__(256) void prefix_table_kernel(uint64_t const *__restrict__ reps,
                                                            int64_t count, int shift,
                                                            int64_t table_size,
                                                            uint32_t *__restrict__ offsets) {
+  if constexpr (!BOUNDED) {
+    int64_t const b = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (b <= table_size)
+      offsets[b] = static_cast<uint32_t>(first_with_prefix(reps, 0, count, shift, static_cast<uint64_t>(b)));
+    return;
+  }
   __shared__ int64_t ends[2];
   int64_t const b0 = static_cast<int64_t>(blockIdx.x) * kPrefixBlock;
   if ((threadIdx.x & 63) == 0 && threadIdx.x < 128)
@@ -149,8 +160,12 @@ bool index_build(IndexData &idx, uint64_t const *d_reps, int64_t count, int numb
   idx.d_reps = d_reps;
   int64_t const table_size = int64_t{1} << prefix_bits;
   if (!idx.d_offsets.allocate(static_cast<size_t>(table_size + 1))) return false;
-  prefix_table_kernel<<<grid_for(table_size + 1, kPrefixBlock), 256, 0, stream()>>>(
-      d_reps, count, idx.shift, table_size, idx.d_offsets.ptr);
+  if (table_size <= kDirectPrefixTable)
+    prefix_table_kernel<false><<<grid_for(table_size + 1, 256), 256, 0, stream()>>>(
+        d_reps, count, idx.shift, table_size, idx.d_offsets.ptr);
+  else
+    prefix_table_kernel<true><<<grid_for(table_size + 1, kPrefixBlock), 256, 0, stream()>>>(
+        d_reps, count, idx.shift, table_size, idx.d_offsets.ptr);
   LSAMD_HIP(hipGetLastError());
   LSAMD_HIP(hipStreamSynchronize(stream()));
   return true;
