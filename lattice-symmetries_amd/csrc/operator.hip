@@ -1339,14 +1339,11 @@ bool build_table_csr(OperatorCore &op, int64_t up, int64_t const *row_ptr, bool 
   LSAMD_HIP(hipMemcpyAsync(h.data(), slots.ptr, sizeof(unsigned long long) * kValueSlots, hipMemcpyDeviceToHost,
                            stream()));
   LSAMD_HIP(hipMemcpyAsync(h_flags, flags.ptr, sizeof(h_flags), hipMemcpyDeviceToHost, stream()));
-  LSAMD_HIP(hipStreamSynchronize(stream()));
-  if (h_flags[1] != 0) { // the general build goes over every pair again and reports what it finds
-    LSAMD_HIP(hipMemsetAsync(op.d_err.ptr, 0, sizeof(int), stream()));
-    many = (h_flags[1] & kManyValues) != 0;
-    return true;
-  }
+  // Waits for the copies.  A pass that stopped early reports what it met, too:
+  // the general build would find the same.
   if (!check_error(op)) return false;
-  if (h_flags[0] == 0) return true;
+  many = (h_flags[1] & kManyValues) != 0;
+  if (h_flags[1] != 0 || h_flags[0] == 0) return true;
   std::vector<std::pair<double, int>> values;
   for (int q = 0; q < kValueSlots; ++q)
     if (h[q] != kEmptySlot) {
