@@ -665,15 +665,15 @@ bool exclusive_scan(uint32_t const *d_counts, int64_t n, uint64_t *d_offsets, ui
 // own least top row, with rows and row pairs of its own that do not fall below
 // its top ones, and the lows that go with it are those of the remaining weight
 // whose rows pass against the top row, listed once per top row and weight.
-// On 6x6 this leaves about one candidate in twenty of the fixed-weight states
-// (before: 4.5 G states, each stepped to by Gosper's rule and tested against
-// its translations), and a candidate costs a list read and one table lookup
+// On 6x6 this leaves 102 M candidates of the 4.5 G states of the sector's weight
+// up to its spin flip (before: each stepped to by Gosper's rule and tested
+// against its translations), and a candidate costs a list read and one table lookup
 // per row pair.  Its survivors (the two top rows are the least pair of the
 // first class) queue up for the full search.  Candidates run in ascending
 // order, so acceptance bits, a scan over tiles and a second pass that writes
 // keep the list ascending.
-// 6x6 basis: 26.7 -> 3.2 ms; the count pass takes 1.9 ms, bound by VALU work and
-// the search's LDS lookups.
+// 6x6 basis: 26.7 -> 3.1 ms; the count pass takes 1.9 to 2.1 ms, bound by VALU work
+// and the search's LDS lookups.
 // ---------------------------------------------------------------------------
 
 constexpr int kSplitTile = 2048; // candidates of a workgroup
@@ -1169,7 +1169,7 @@ bool enumerate_states(EnumerationSpec const &spec, uint64_t lower, uint64_t uppe
   bool const use_factored = q_identity >= 0;
   // The split enumeration lists the whole sector's candidates, so it serves
   // ranges of at least an eighth of the sector (it does about a tenth of the
-  // filter's work: 3.2 against 26.7 ms on 6x6) where it pays.
+  // filter's work: 3.1 against 26.7 ms on 6x6) where it pays.
   if (use_factored && g.lines() && split_low_rows(g) > 0 &&
       static_cast<uint64_t>(p.total) >= binomial_host(n, p.hamming) / (spec.spin_inversion != 0 ? 16 : 8) &&
       (split_pays(g, p.total) || g_factored_enumeration.load() == 2)) {

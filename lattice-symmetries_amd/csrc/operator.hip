@@ -231,10 +231,11 @@ inline size_t terms_lds_bytes(int T) { return static_cast<size_t>(T) * 16; }
 // one or two terms on neighbouring rows: their targets lie close together, so
 // the index lookups and the atomics share cache lines.  Listing a row's pairs
 // together instead spreads every wave over the whole basis: 57 against 43 ms
-// for the CSR fill on 6x6 and 2.04 against 1.86 ms for the 32-site chain's
-// on-the-fly product (one lane to a row: 81 ms without the counting atomics,
-// and 1.86 ms).  Bound by the cache lines that miss L2 under the lookups and
-// atomics (42 G random atomics/s reach the basis) as much as by the search.
+// for the CSR fill on 6x6.  One lane to a row: 81 ms there without the counting
+// atomics, and 1.92 against 1.75 ms for the 32-site chain's on-the-fly product.
+// The 6x6 fill issues 1.7e10 VALU instructions (28 of its 43 ms) and misses L2
+// 1.77 G times under lookups and counting atomics (41 G/s; random atomics alone
+// reach the basis at 42 G/s), so it is bound by both.
 constexpr int kPairThreads = 256;
 constexpr int kWaveRows = 64;
 constexpr int kPairTermBits = 13; // of a term and of a pair's rank in its row
@@ -247,7 +248,16 @@ struct WaveRows {
 };
 constexpr size_t kPairLds = sizeof(WaveRows) * (kPairThreads / 64);
 
-// Rows of a wave: enough waves for the chip first.
+// Rows of a wave: enough waves for the chip first; more rows share more cache
+// lines, fewer leave less to the last waves.  Where the line lies depends on the
+// cost of a pair.  On-the-fly product, ms at 4, 8, 16, 32, 64 rows:
+//   107 k rows (6x6, weight 8)   0.59 0.54 0.60 1.00 1.90   (16 taken)
+//   330 k rows (6x6, weight 9)   1.34 1.20 1.17 1.22 1.84   (64)
+//   718 k rows (28-site chain)   0.65 0.58 0.54 0.55 0.55   (64)
+//   4.4 M rows (6x6, weight 12)  12.7 11.2 10.5 10.2 10.2   (64)
+// Doubling at 49 152 rows a step instead would win 6x6 with weight 9 (1.20 ms)
+// and lose without an orbit search (185 k states of 20 sites, all pairs: 0.28 ->
+// 0.37 ms, its CSR build 0.89 -> 1.06).
 inline int wave_rows(int64_t n) {
   int rows = 4;
   while (rows < kWaveRows && n >= int64_t{8192} * rows) rows *= 2;
@@ -893,7 +903,7 @@ __global__ __launch_bounds__(64) void sort_rows_kernel(int64_t n, int64_t const 
 // Rows of at most kShortRow entries, one wave per row, in registers: entry
 // 64 e + lane of the padded row in v[e], a bitonic network over swizzles for
 // distances below 64 and within the lane above; which lanes keep the smaller
-// key is a constant of the step.  VALU-bound: 6.2 ms for the 15.8 M rows of
+// key is a constant of the step.  VALU-bound: 6.0 ms for the 15.8 M rows of
 // 6x6 (74 entries each), against 24 ms with 64-bit keys in LDS (barriers and
 // LDS round trips in every step).
 constexpr int kShortRow = 256;
@@ -1310,7 +1320,7 @@ __global__ __launch_bounds__(256) void split_wide_keys_kernel(int64_t nnz, uint6
 // writes, and a sort of 6 ms replace a counting pass (28 ms), a scatter of
 // 8-byte keys through atomic cursors (42 ms), their LDS sort (24 ms), a gather
 // of the values in target order (23 ms), the distinct-value pass and the
-// packing (11 ms), and the temporaries shrink from 28 to 14 GB.  `done` stays
+// packing (9 ms), and the temporaries shrink from 28 to 14 GB.  `done` stays
 // false when the matrix has too many values (`many`), a target row of more than
 // 4096 entries, or no entries: then the general build runs.
 bool build_table_csr(OperatorCore &op, int64_t up, int64_t const *row_ptr, bool &done, bool &many) {
@@ -1405,9 +1415,11 @@ bool build_table_csr(OperatorCore &op, int64_t up, int64_t const *row_ptr, bool 
 // The product schedule when neither the caller nor the autotuner chose one:
 // lanes per row so that each lane sums about four entries of a mean row, and
 // for a million rows or more the die-aware mapping with one workgroup per
-// tile, the autotuner's choice for such matrices (16 lanes and that mapping
-// on 6x6, against 8 lanes on the plain grid otherwise; the FP32 block of 8
-// takes 9.2 ms with it and 10.2 on the plain grid).
+// tile, the autotuner's choice on 6x6 (16 lanes and that mapping).  Plain against
+// die-aware grid, ms: FP32 block of 8 at 0.36 M rows 0.062 / 0.062, 0.72 M
+// 0.123 / 0.112, 0.89 M (59 entries a row) 0.376 / 0.342, 1.3 M 0.244 / 0.223,
+// 4.7 M 0.893 / 0.870, 15.8 M (6x6) 10.2 / 9.2.  The FP64 vector gains only where
+// x outgrows the caches: 1.3 M 0.114 / 0.129, 4.4 M 1.59 / 1.67.
 void default_schedule(OperatorCore &op) {
   Csr const &c = op.csr;
   double const mean = c.rows > 0 ? static_cast<double>(c.nnz) / static_cast<double>(c.rows) : 0.0;

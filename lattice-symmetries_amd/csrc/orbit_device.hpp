@@ -471,8 +471,9 @@ template <int SI> __device__ __forceinline__ double free_orbit_norm(GroupView co
 // 96 row lookups and the divergent loops that formed every image with the
 // least top row, and the images in x's own class for the stabiliser sum:
 // state_info of the 15.8 M representatives takes 0.50 ms against 1.87 ms
-// (state_info_factored), the CSR fill's 1.17 G searches 81 ms against 181 ms.
-// Bound by VALU and LDS lookups in the first part, by divergence over the
+// (state_info_factored); the CSR fill's 1.17 G searches, index lookups and
+// counting atomics take 43 ms, the pairs dealt to lanes (181 ms with
+// state_info_factored, one lane to a row and no atomics).  Bound by VALU and LDS lookups in the first part, by divergence over the
 // images that are formed in the second.
 template <typename W, int SI> struct LineSearch {
   W *base, *kept;       // LDS: images of rows under the class bases; one base image per lane and class
@@ -577,8 +578,9 @@ template <typename W, int SI> struct LineSearch {
 // top are formed.  rotl(z, L) & rotl(z, L - 1) & .. & z leaves one bit at the
 // top end of every run of at least L + 1 zeros.  On the 32-site chain (64
 // elements with parity, flipped copies too) about 5 such steps and 2 images
-// per word replace 32 rotations: the on-the-fly product takes 1.92 ms against
-// 5.77 ms with all rotations formed.  Bound by VALU work; a word per point
+// per word replace 32 rotations: the on-the-fly product takes 1.75 ms against
+// 5.76 ms with all rotations formed (one lane to a row; 1.92 ms so with this
+// search).  Bound by VALU work; a word per point
 // element and flip is kept in LDS, so at most kMaxRunPoints of them.
 template <typename W, int D, int SI> struct RunSearch {
   static constexpr int kFlips = SI != 0 ? 2 : 1;
@@ -648,8 +650,8 @@ template <typename W, int D, int SI> struct RunSearch {
 // the up state are formed.  Signs come from a bit table per species: the
 // species do not pass each other.  On the 4x4 Hubbard sector (128 elements)
 // this replaces 128 networks of 9 stages per state: the complex on-the-fly
-// product takes 1.7 ms against 11.8 ms, now bound by its atomics (42 G/s), and
-// the norms 0.02 ms.
+// product takes 1.68 ms against 13.6 ms (11.8 ms element by element with the
+// pairs dealt to lanes), now bound by its atomics (42 G/s), and the norms 0.02 ms.
 template <typename W, int D> struct SpeciesSearch {
   W *masks; // LDS: the networks, element-major
   double norm_1;

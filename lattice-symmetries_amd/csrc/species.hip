@@ -4,11 +4,11 @@
 // sites of both species alike, so an image is (e(down), e(up)) and the least
 // one has the least image of `down`.  For at most 16 sites the least image of
 // every species state, the elements that reach it and the sign of every
-// element on every species state fit tables of about 2 MB, which take 0.2 ms
-// to make.  With them the 4x4 basis of 7 + 7 fermions (131 M products, 1.02 M
+// element on every species state fit tables of about 2 MB, which take 0.16 ms
+// of kernels to make.  With them the 4x4 basis of 7 + 7 fermions (131 M products, 1.02 M
 // representatives) lists the down states that are their own least image and
-// tests 1.3 M products: 3.2 -> 0.9 ms, most of it launches and copies of a few
-// KB.
+// tests 1.3 M products: 3.3 -> 0.54 ms with the making of group and tables, 0.4 ms
+// where those are there, most of it launches and copies of a few KB.
 #include <algorithm>
 
 #include "orbit_device.hpp"
